@@ -55,6 +55,9 @@ def common_flags() -> list[str]:
         f"--offload-arch={ARCH}",
         "-ffp-contract=off",
         "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+        # MFMA results in VGPRs: the kernels' VALU consumes them at once, and a
+        # copy out of an AGPR would cost an instruction per value.
+        "-mllvm", "-amdgpu-mfma-vgpr-form=1",
         "-I", str(ROOT / "include"),
         "-Wall", "-Wno-unused-result",
     ]

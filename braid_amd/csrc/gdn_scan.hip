@@ -1,14 +1,15 @@
 // Batched Gated DeltaNet decode step and chunk prefill scan for gfx950.
 //
-// Both kernels launch one workgroup per (batch row, value head) tile and run
-// the same per-token arithmetic with the same summation trees: decode with
-// four waves of 32 state rows x 128 columns (gdn_token, column sums finished
-// across waves in LDS), prefill with four waves of 128 rows x 32 columns
-// (scan_token, column sums finished inside each wave, no barrier per token).
-// Decode loads the tile from the slot-indexed pool, runs one token and stores
-// it back; prefill loads it once, runs T tokens with the tile resident in
-// registers (in the pool's storage type) and stores it once. Reference behaviour: braid/kernels/csrc/gdn_decode.cu:156-272 (decode)
-// and :467-551 (prefill); entry-point contracts :313-441 and :553-699.
+// Decode launches one workgroup of four waves per (batch row, value head) tile
+// (or column part of it): it loads the tile from the slot-indexed pool, runs
+// one token and stores it back. Prefill loads a tile's columns once, runs T
+// tokens with them resident in registers (in the pool's storage type) and
+// stores them once; no column sum leaves a wave, so no token needs a barrier.
+// fp32 pools run gdn_tile.h's VALU token in both, 16-bit pools the matrix-core
+// token (gdn_mfma.h for decode, gdn_scan16.h for prefill); either way a chunk
+// equals its decode steps bit for bit. Reference behaviour:
+// braid/kernels/csrc/gdn_decode.cu:156-272 (decode) and :467-551 (prefill);
+// entry-point contracts :313-441 and :553-699.
 #include <algorithm>
 #include <cmath>
 #include <deque>
@@ -23,6 +24,8 @@
 
 #include "capi_common.h"
 #include "conv_common.h"
+#include "gdn_mfma.h"
+#include "gdn_scan16.h"
 #include "gdn_tile.h"
 #include "stream_shape.h"
 
@@ -34,9 +37,8 @@ namespace {
 // P column parts: the tile's 128 columns are split over P workgroups of four
 // waves, part p owning columns [128 p / P, 128 (p + 1) / P) with 8 / P columns
 // per lane. Every column sum runs over rows within the column, so a part
-// needs nothing from the others: each lane keeps the same eight rows and its
-// chains, the row-group butterfly and the cross-wave tree are unchanged, and
-// the results are the one-part layout's bits. Small launches use 2 or 4 parts
+// needs nothing from the others: each lane keeps the same eight rows, its
+// columns' sums are unchanged, and the results are the one-part layout's bits. Small launches use 2 or 4 parts
 // to spread each tile's arithmetic over more CUs (its latency is the
 // per-lane work, which shrinks with the columns). fp32 pools split a lane's
 // columns into two runs 64 apart only with one part.
@@ -44,8 +46,21 @@ namespace {
 // kWavesPerSimd bounds the register budget: 4 (128 VGPRs) where up to four
 // workgroups share a CU; 2 for the large launches that stream_shape caps at
 // two workgroups per CU, where 256 VGPRs cost no residency and the compiler
-// schedules the prologue's loads more freely (169 VGPRs; B = 128: 47.92 ->
-// 47.63 us a step in one A/B run).
+// schedules the prologue's loads more freely (B = 128: 47.92 -> 47.63 us a step
+// in one A/B run). With the sums on the matrix cores a 16-bit pool's step at B =
+// 128 takes 47.1 us (47.4 with VALU chains and butterflies), B = 64 25.8 (26.1),
+// B = 8 5.0 (5.2), fp16, graph of 48 launches.
+template <class Tag>
+struct DecodeLds {  // a decode workgroup's LDS, by token kernel
+  using Tile = TileLds16;
+  using QKWave = QKParts<Tag>;
+};
+template <>
+struct DecodeLds<F32> {
+  using Tile = TileLds;
+  using QKWave = QKLds;
+};
+
 template <class Tag, class Gates, int P, int kWavesPerSimd = 4>
 __global__ void __launch_bounds__(tile_threads(kDecodeCols))
 __attribute__((amdgpu_waves_per_eu(1, kWavesPerSimd)))
@@ -73,8 +88,8 @@ gdn_decode_kernel(typename Storage<Tag>::T* __restrict__ pool, const int* __rest
   const int h = tix - b * H;
   const int g = h / heads_per_group;
   const LaneMap<CPL, std::is_same<Tag, F32>::value && P == 1> L(threadIdx.x, part);
-  __shared__ TileLds lds;
-  __shared__ QKLds qk_lds[kWaves];
+  __shared__ typename DecodeLds<Tag>::Tile lds;
+  __shared__ typename DecodeLds<Tag>::QKWave qk_lds[kWaves];
 
   // Reads in issue order: the slot (the slot map lives in device memory, so
   // one captured graph serves any slot assignment, gdn_decode.cu:230-236);
@@ -110,20 +125,30 @@ gdn_decode_kernel(typename Storage<Tag>::T* __restrict__ pool, const int* __rest
   // Every wave holds the gate inputs here, so their reads stay where they
   // were issued rather than moving into the wave that evaluates each gate.
   Gates::keep(gin);
-  publish_gates(L, gates, gates.raw_of(gin), gates.consts_of(gin), lds);
-  QK qk;
-  normalize_qk_lds(L, q2, k2, qk_lds[L.wave], qk);
-
-  float yy[CPL];
-  // Row-group sums through the permlane swaps, not the LDS crossbar: this
-  // kernel has the registers, and a B = 128 step gains 0.66 us (48.48 ->
-  // 47.82) from the shorter per-tile chain.
-  gdn_token<Tag, CPL, true>(L, S, qk, vv, lds, yy);
-
+  publish_gates(L, gates, gates.raw_of(gin), gates.consts_of(gin), lds.gate);
+  float* const y_row = y + ((size_t)b * H + h) * kHD;
+  auto store_state = [&] {
 #pragma unroll
-  for (int i = 0; i < kRowsPerLane; ++i) store_row(S[i], L, tile + (size_t)L.row(i) * kHD);
-  // Each column's totals sit in all lanes of its chunk; one lane per chunk writes them.
-  if (L.stores_y()) store_cols(L, y + ((size_t)b * H + h) * kHD, yy);
+    for (int i = 0; i < kRowsPerLane; ++i) store_row(S[i], L, tile + (size_t)L.row(i) * kHD);
+  };
+  if constexpr (std::is_same<Tag, F32>::value) {
+    QK qk;
+    normalize_qk_lds(L, q2, k2, qk_lds[L.wave], qk);
+    // Row-group sums through the permlane swaps, not the LDS crossbar: this
+    // kernel has the registers, and the per-tile chain is shorter.
+    float yy[CPL];
+    gdn_token<Tag, CPL, true>(L, S, qk, vv, lds, yy);
+    store_state();
+    // Each column's totals sit in all lanes of its chunk; one lane per chunk writes them.
+    if (L.stores_y()) store_cols(L, y_row, yy);
+  } else {
+    QKOps<Tag> qk;
+    split_qk_lds<Tag>(L, q2, k2, qk_lds[L.wave], qk);
+    float delta[CPL];
+    gdn_token16<Tag, CPL>(L, S, qk, vv, lds, delta);
+    store_state();
+    token16_readout<Tag, CPL>(L, qk, lds, delta, y_row);
+  }
 }
 
 // The conv1d decode step fused into the GDN decode step (one launch for the
@@ -137,10 +162,11 @@ gdn_decode_kernel(typename Storage<Tag>::T* __restrict__ pool, const int* __rest
 // conv1d_decode followed by gdn_decode, bit for bit. A group's q/k windows are
 // advanced once because one workgroup owns all heads that read them. The conv
 // outputs never go to memory: nothing but the recurrence reads them.
-template <int HPG>
+template <class Tag, int HPG>
 struct ConvDecodeLds {
-  TileLds tile[HPG];
+  typename DecodeLds<Tag>::Tile tile[HPG];
   float qkv[2 + HPG][kHD];  // conv outputs: q, k, then each head's v
+  typename DecodeLds<Tag>::QKWave qk[std::is_same<Tag, F32>::value ? 1 : HPG * kWaves];
 };
 
 // The decode token of tile t of a conv + decode workgroup, on the conv
@@ -148,19 +174,33 @@ struct ConvDecodeLds {
 template <class Tag, int HPG, class LM>
 __device__ __forceinline__ void decode_token_from_lds(const LM& L,
                                                       Row<Tag, kDecodeCols> (&S)[kRowsPerLane],
-                                                      ConvDecodeLds<HPG>& lds, int t,
+                                                      ConvDecodeLds<Tag, HPG>& lds, int t,
                                                       typename Storage<Tag>::T* tile,
                                                       float* y_row) {
   constexpr int CPL = kDecodeCols;
   float vv[CPL];
   load_cols(L, lds.qkv[2 + t], vv);
-  QK qk;
-  normalize_qk(L, lds.qkv[0], lds.qkv[1], qk);
-  float yy[CPL];
-  gdn_token<Tag, CPL>(L, S, qk, vv, lds.tile[t], yy);
+  auto store_state = [&] {
 #pragma unroll
-  for (int i = 0; i < kRowsPerLane; ++i) store_row(S[i], L, tile + (size_t)L.row(i) * kHD);
-  if (L.stores_y()) store_cols(L, y_row, yy);
+    for (int i = 0; i < kRowsPerLane; ++i) store_row(S[i], L, tile + (size_t)L.row(i) * kHD);
+  };
+  if constexpr (std::is_same<Tag, F32>::value) {
+    QK qk;
+    normalize_qk(L, lds.qkv[0], lds.qkv[1], qk);
+    float yy[CPL];
+    gdn_token<Tag, CPL>(L, S, qk, vv, lds.tile[t], yy);
+    store_state();
+    if (L.stores_y()) store_cols(L, y_row, yy);
+  } else {
+    float2 q2, k2;
+    load_qk2(L, lds.qkv[0], lds.qkv[1], q2, k2);
+    QKOps<Tag> qk;
+    split_qk_lds<Tag>(L, q2, k2, lds.qk[t * kWaves + L.w], qk);
+    float delta[CPL];
+    gdn_token16<Tag, CPL>(L, S, qk, vv, lds.tile[t], delta);
+    store_state();
+    token16_readout<Tag, CPL>(L, qk, lds.tile[t], delta, y_row);
+  }
 }
 
 template <class Tag, class XT, class Gates, int HPG>
@@ -190,7 +230,7 @@ __device__ __forceinline__ void conv_decode_body(typename Storage<Tag>::T* __res
   const int h = g * HPG + t;
   const LaneMap<CPL, std::is_same<Tag, F32>::value> L(threadIdx.x % kTileThreads);
 
-  __shared__ ConvDecodeLds<HPG> lds;
+  __shared__ ConvDecodeLds<Tag, HPG> lds;
 
   // The group's conv channels: segment 0 = q (channels g*SS..), 1 = k
   // (G*SS + g*SS..), 2 + j = v of head g*HPG + j (2*G*SS + head*HD..).
@@ -254,7 +294,7 @@ __device__ __forceinline__ void conv_decode_body(typename Storage<Tag>::T* __res
         store_window<kK>(win + (unsigned)c * kK, w[m]);
       }
     }
-    publish_gates(L, gates, gates.raw_of(gin), gates.consts_of(gin), lds.tile[t]);
+    publish_gates(L, gates, gates.raw_of(gin), gates.consts_of(gin), lds.tile[t].gate);
     __syncthreads();
     decode_token_from_lds<Tag, HPG>(L, S, lds, t, tile, y + ((size_t)b * H + h) * kHD);
   } else {
@@ -273,7 +313,7 @@ __device__ __forceinline__ void conv_decode_body(typename Storage<Tag>::T* __res
     }
     __syncthreads();
     publish_gates(L, gates, gates.load(b, h, 0, H, 1), GateConst{gates.A[h], gates.dt_bias[h]},
-                  lds.tile[t]);
+                  lds.tile[t].gate);
     decode_token_from_lds<Tag, HPG>(L, S, lds, t, tile, y + ((size_t)b * H + h) * kHD);
   }
 }
@@ -304,7 +344,9 @@ gdn_conv_decode_kernel_f32(float* __restrict__ pool, float* __restrict__ conv_po
                                         H, G, C);
 }
 
-// A prefill stage: the next kStage tokens' per-token inputs, staged in LDS by
+// The fp32 pool's prefill.
+//
+// A stage: the next kStage tokens' per-token inputs, staged in LDS by
 // a parallel prologue so that the serial loop reads nothing from global memory:
 //   qk   normalised q and k (q_hat, k_hat), each kStageVec floats holding the
 //        kSS rows in the order the launch's layout reads them (StageOrder);
@@ -572,9 +614,8 @@ __device__ __forceinline__ void read_token_eighth(const StageLds& st, int j, int
 
 // The eighth layout's state: the lane's chain, rows i = 2m and 2m + 1 in
 // p[m].
-template <class Tag>
 struct ScanStateE {
-  RowPair1<Tag> p[kRowsPerLane / 2];
+  RowPair1 p[kRowsPerLane / 2];
   template <class ST>
   __device__ __forceinline__ void load(const ScanMapEighth& L, const ST* tile) {
 #pragma unroll
@@ -589,25 +630,25 @@ struct ScanStateE {
   }
 };
 
-template <class Tag, int CPL, int kLRG>
+template <int CPL, int kLRG>
 struct ScanState;
 
 // One token of a ScanMap layout (one or two columns per lane) on its state.
-template <class Tag, int CPL, bool kOpaqueNarrow = false>
-__device__ __forceinline__ void scan_token_any(ScanState<Tag, CPL, kRowGroups>& S,
+template <int CPL>
+__device__ __forceinline__ void scan_token_any(ScanState<CPL, kRowGroups>& S,
                                                const TokenIn<CPL>& in, float (&y)[CPL]) {
   if constexpr (CPL == 1)
-    scan_token_pairs<Tag, kOpaqueNarrow>(S.p, in.kh, in.qh, in.v[0], in.alpha, in.beta, y[0]);
+    scan_token_pairs(S.p, in.kh, in.qh, in.v[0], in.alpha, in.beta, y[0]);
   else
-    scan_token<Tag, CPL, kOpaqueNarrow>(S.s, in.kh, in.qh, in.v, in.alpha, in.beta, y);
+    scan_token<CPL>(S.s, in.kh, in.qh, in.v, in.alpha, in.beta, y);
 }
 
 // A lane's state in a scan layout: a Row<Tag, CPL> per (row group, i), or,
 // with one column per lane, row pairs (RowPair1) over row groups 2p and 2p + 1
 // so that one packed conversion narrows two elements.
-template <class Tag, int CPL, int kLRG>
+template <int CPL, int kLRG>
 struct ScanState {
-  Row<Tag, CPL> s[kLRG][kRowsPerLane];
+  Row<F32, CPL> s[kLRG][kRowsPerLane];
   template <class LM, class ST>
   __device__ __forceinline__ void load(const LM& L, const ST* tile) {
 #pragma unroll
@@ -625,9 +666,9 @@ struct ScanState {
     }
   }
 };
-template <class Tag, int kLRG>
-struct ScanState<Tag, 1, kLRG> {
-  RowPair1<Tag> p[kLRG / 2][kRowsPerLane];
+template <int kLRG>
+struct ScanState<1, kLRG> {
+  RowPair1 p[kLRG / 2][kRowsPerLane];
   template <class LM, class ST>
   __device__ __forceinline__ void load(const LM& L, const ST* tile) {
 #pragma unroll
@@ -667,8 +708,8 @@ struct ScanState<Tag, 1, kLRG> {
 // into +0. y at the pad positions [len, T) is written as 0 (the reference
 // leaves arbitrary values there that nothing reads; zeros also keep a later
 // per-tensor FP8 scale of the readout independent of the pads).
-template <class Tag, class Gates, int Layout, bool kTokenPairs = false>
-__device__ __forceinline__ void prefill_tile(typename Storage<Tag>::T* __restrict__ pool,
+template <class Gates, int Layout, bool kTokenPairs = false>
+__device__ __forceinline__ void prefill_tile(float* __restrict__ pool,
                                              const int* __restrict__ slot_idx,
                                              const float* __restrict__ q,
                                              const float* __restrict__ k,
@@ -679,13 +720,12 @@ __device__ __forceinline__ void prefill_tile(typename Storage<Tag>::T* __restric
   using LM = typename ScanLayoutOf<Layout>::type;
   constexpr int CPL = LM::kCPL;
   constexpr int kLRG = LM::kLaneRowGroups;
-  using ST = typename Storage<Tag>::T;
   const int g = h / heads_per_group;
   const LM L(threadIdx.x, part);
   const int slot = slot_idx[b];
-  ST* tile = pool + ((size_t)slot * H + h) * (kSS * kHD) + L.col0;
+  float* tile = pool + ((size_t)slot * H + h) * (kSS * kHD) + L.col0;
 
-  typename std::conditional<Layout == 8, ScanStateE<Tag>, ScanState<Tag, CPL, kLRG>>::type S;
+  typename std::conditional<Layout == 8, ScanStateE, ScanState<CPL, kLRG>>::type S;
   S.load(L, tile);
 
   constexpr int kW = LM::kWaves;
@@ -723,8 +763,8 @@ __device__ __forceinline__ void prefill_tile(typename Storage<Tag>::T* __restric
       auto clamp = [](int t) { return min(t, kStage - 1); };
       auto pair = [&](int jj, const TokenInE& a, const TokenInE& c) {
         float y0[1], y1[1];
-        scan_token_eighth<Tag, true>(S.p, a.kh, a.qh, a.v, a.alpha, a.beta, y0[0]);
-        scan_token_eighth<Tag, true>(S.p, c.kh, c.qh, c.v, c.alpha, c.beta, y1[0]);
+        scan_token_eighth(S.p, a.kh, a.qh, a.v, a.alpha, a.beta, y0[0]);
+        scan_token_eighth(S.p, c.kh, c.qh, c.v, c.alpha, c.beta, y1[0]);
         if (L.stores_y()) {
           storeN<1>(yt + jj * y_tok, y0);
           storeN<1>(yt + (jj + 1) * y_tok, y1);
@@ -749,7 +789,7 @@ __device__ __forceinline__ void prefill_tile(typename Storage<Tag>::T* __restric
       }
       if (j < n) {
         float yy[1];
-        scan_token_eighth<Tag>(S.p, c0.kh, c0.qh, c0.v, c0.alpha, c0.beta, yy[0]);
+        scan_token_eighth(S.p, c0.kh, c0.qh, c0.v, c0.alpha, c0.beta, yy[0]);
         if (L.stores_y()) storeN<1>(yt + j * y_tok, yy);
       }
     } else if constexpr (Layout == 4) {
@@ -759,9 +799,9 @@ __device__ __forceinline__ void prefill_tile(typename Storage<Tag>::T* __restric
           read_token_quarter(st, j, r0, L.col0, in0);
           read_token_quarter(st, j + 1, r0, L.col0, in1);
           float y0[1], y1[1];
-          scan_token_quarter<Tag, true>(S.p[0], in0.kh, in0.qh, in0.v, in0.alpha, in0.beta,
+          scan_token_quarter(S.p[0], in0.kh, in0.qh, in0.v, in0.alpha, in0.beta,
                                         y0[0]);
-          scan_token_quarter<Tag, true>(S.p[0], in1.kh, in1.qh, in1.v, in1.alpha, in1.beta,
+          scan_token_quarter(S.p[0], in1.kh, in1.qh, in1.v, in1.alpha, in1.beta,
                                         y1[0]);
           if (L.stores_y()) {
             storeN<1>(yt + j * y_tok, y0);
@@ -773,7 +813,7 @@ __device__ __forceinline__ void prefill_tile(typename Storage<Tag>::T* __restric
         TokenInQ in;
         read_token_quarter(st, j, r0, L.col0, in);
         float yy[1];
-        scan_token_quarter<Tag>(S.p[0], in.kh, in.qh, in.v, in.alpha, in.beta, yy[0]);
+        scan_token_quarter(S.p[0], in.kh, in.qh, in.v, in.alpha, in.beta, yy[0]);
         if (L.stores_y()) storeN<1>(yt + j * y_tok, yy);
       }
     } else if constexpr (kTokenPairs) {
@@ -792,8 +832,8 @@ __device__ __forceinline__ void prefill_tile(typename Storage<Tag>::T* __restric
         read_token<CPL>(st, j, r0, L.col0, in0);
         read_token<CPL>(st, j + 1, r0, L.col0, in1);
         float y0[CPL], y1[CPL];
-        scan_token_any<Tag, CPL, true>(S, in0, y0);
-        scan_token_any<Tag, CPL, true>(S, in1, y1);
+        scan_token_any<CPL>(S, in0, y0);
+        scan_token_any<CPL>(S, in1, y1);
         if (L.stores_y()) {
           storeN<CPL>(yt + j * y_tok, y0);
           storeN<CPL>(yt + (j + 1) * y_tok, y1);
@@ -805,7 +845,7 @@ __device__ __forceinline__ void prefill_tile(typename Storage<Tag>::T* __restric
         TokenIn<CPL> in;
         read_token<CPL>(st, j, r0, L.col0, in);
         float yy[CPL];
-        scan_token_any<Tag, CPL>(S, in, yy);
+        scan_token_any<CPL>(S, in, yy);
         if (L.stores_y()) storeN<CPL>(yt + j * y_tok, yy);
       }
     }
@@ -826,7 +866,8 @@ __device__ __forceinline__ void prefill_tile(typename Storage<Tag>::T* __restric
   }
 }
 
-// A scan wave issues at most one VALU instruction per about five clocks and
+// Scan waves of both kinds run at the highest wave priority. A wave issues at
+// most one VALU instruction per about five clocks and
 // waits on its own dependency chains between them, so its SIMD has issue
 // cycles to spare. A decode launched beside it (MixedTick: a memory-bound
 // launch on a side stream) shares those SIMDs; at the highest wave priority
@@ -839,10 +880,9 @@ __device__ __forceinline__ void raise_scan_priority() { __builtin_amdgcn_s_setpr
 // (layout 4, kParts = 4) or an eighth (layout 8, kParts = 8) per workgroup:
 // blockIdx.x = (b * H + h) * kParts + part. Layouts 1, 4 and 8 run token
 // pairs.
-template <class Tag, class Gates, int Layout>
+template <class Gates, int Layout>
 __global__ void __launch_bounds__(64 * ScanLayoutOf<Layout>::type::kWaves)
-gdn_prefill_kernel(typename Storage<Tag>::T* __restrict__ pool,
-                   const int* __restrict__ slot_idx,
+gdn_prefill_kernel(float* __restrict__ pool, const int* __restrict__ slot_idx,
                    const float* __restrict__ q, const float* __restrict__ k,
                    const float* __restrict__ v, Gates gates, float* __restrict__ y,
                    int H, int G, int heads_per_group, int T) {
@@ -853,12 +893,156 @@ gdn_prefill_kernel(typename Storage<Tag>::T* __restrict__ pool,
   const int b = tile_id / H;
   const int h = tile_id - b * H;
   __shared__ StageLds st;
-  prefill_tile<Tag, Gates, Layout, Layout != 2>(pool, slot_idx, q, k, v, gates, y, H, G,
+  prefill_tile<Gates, Layout, Layout != 2>(pool, slot_idx, q, k, v, gates, y, H, G,
                                                 heads_per_group, T, b, h, part,
                                                 gates.row_len(b, T), st);
 }
 
-// Ragged batches of up to four tiles per CU: the rows' live lengths decide
+template <class Tag, class Gates, int Layout>
+__global__ void __launch_bounds__(Scan16Map<Layout>::kThreads)
+gdn_prefill16_kernel(uint16_t* __restrict__ pool, const int* __restrict__ slot_idx,
+                     const float* __restrict__ q, const float* __restrict__ k,
+                     const float* __restrict__ v, Gates gates, float* __restrict__ y, int H, int G,
+                     int heads_per_group, int T) {
+  constexpr int kParts = Scan16Map<Layout>::kParts;
+  raise_scan_priority();
+  const int tile_id = blockIdx.x / kParts;
+  const int part = blockIdx.x - tile_id * kParts;
+  const int b = tile_id / H;
+  const int h = tile_id - b * H;
+  __shared__ Scan16Lds<Tag, Layout> lds;
+  prefill_tile16<Tag, Gates, Layout>(pool, slot_idx, q, k, v, gates, y, H, G, heads_per_group, T,
+                                     b, h, part, gates.row_len(b, T), lds);
+}
+
+// A token's time in each tier of the planned kernel, us (MI355X, one workgroup
+// per CU, 384-token rows; tiers 0 eighth, 1 quarter, 2 split, 3 whole).
+struct TierTimes {
+  float us[4];
+};
+template <class Tag>
+__host__ __device__ constexpr TierTimes tier_times() {
+  if (std::is_same<Tag, F16>::value) return {{0.160f, 0.172f, 0.250f, 0.392f}};
+  return {{0.193f, 0.240f, 0.375f, 0.560f}};
+}
+constexpr int kMaxPlanRows = 1024;
+// Bounds of a plan's upgraded rows.
+constexpr int kMaxN8 = 2, kMaxN4 = 6, kMaxN2 = 8;
+constexpr int kPlans = (kMaxN8 + 1) * (kMaxN4 + 1) * (kMaxN2 + 1);
+
+// Ragged batches on a 16-bit pool: each row runs in a tier by its rank in
+// length (the n8 longest eighth, the next n4 quarter, the next n2 split, the
+// rest whole), workgroups in the order of their durations, longest first, so
+// that the long ones start on CUs of their own and the short ones fill in (a
+// CU holds one workgroup: twelve waves of up to 168 registers). plan: the
+// host's choice, n8 * 2^20 + n4 * 2^10 + n2, or -1 (a captured call without
+// host lengths): every workgroup then takes the plan that minimises the larger
+// of its longest row's time and its total time over the CUs, within max_extra
+// workgroups beyond one per tile (what the grid has room for). The grid's
+// workgroups beyond the plan return. A row's bits do not depend on its tier.
+template <class Tag, class Gates>
+__global__ void __launch_bounds__(Scan16Map<2>::kThreads)
+gdn_prefill16_planned_kernel(uint16_t* __restrict__ pool, const int* __restrict__ slot_idx,
+                             const float* __restrict__ q, const float* __restrict__ k,
+                             const float* __restrict__ v, Gates gates, float* __restrict__ y,
+                             int B, int H, int G, int heads_per_group, int T, int cus,
+                             int max_extra, int plan) {
+  raise_scan_priority();
+  union Lds {
+    Scan16Lds<Tag, 1> l1;
+    Scan16Lds<Tag, 2> l2;
+    Scan16Lds<Tag, 4> l4;
+    Scan16Lds<Tag, 8> l8;
+  };
+  struct Plan {
+    int len[kMaxPlanRows];    // by row
+    int order[kMaxPlanRows];  // row of each rank in length
+    unsigned long long best;  // the least (estimate, plan)
+    int row, tier, first;     // this workgroup's
+  };
+  // The plan's scratch and the tile's stages in the same memory.
+  __shared__ alignas(16) char smem[sizeof(Lds) > sizeof(Plan) ? sizeof(Lds) : sizeof(Plan)];
+  Plan& ps = *reinterpret_cast<Plan*>(smem);
+  const int nt = blockDim.x, tid = threadIdx.x;
+  constexpr int kTierParts[4] = {8, 4, 2, 1};
+  const TierTimes tt = tier_times<Tag>();
+  for (int r = tid; r < B; r += nt) ps.len[r] = gates.row_len(r, T);
+  if (tid == 0) {
+    ps.best = ~0ull;
+    ps.row = -1;
+  }
+  __syncthreads();
+  for (int r = tid; r < B; r += nt) {
+    int rank = 0;
+    for (int o = 0; o < B; ++o)
+      rank += (ps.len[o] > ps.len[r] || (ps.len[o] == ps.len[r] && o < r)) ? 1 : 0;
+    ps.order[rank] = r;
+  }
+  __syncthreads();
+  if (plan < 0) {
+    if (tid < kPlans) {
+      const int n8 = tid / ((kMaxN4 + 1) * (kMaxN2 + 1)), n4 = tid / (kMaxN2 + 1) % (kMaxN4 + 1),
+                n2 = tid % (kMaxN2 + 1);
+      if (n8 + n4 + n2 <= B && (7 * n8 + 3 * n4 + n2) * H <= max_extra) {
+        float longest = 0.f, work = 0.f;
+        for (int r = 0; r < B; ++r) {
+          const int t = r < n8 ? 0 : (r < n8 + n4 ? 1 : (r < n8 + n4 + n2 ? 2 : 3));
+          const float us = tt.us[t] * (float)ps.len[ps.order[r]];
+          longest = fmaxf(longest, us);
+          work += us * (float)kTierParts[t];
+        }
+        const float est = fmaxf(longest, work * (float)H / (float)cus);
+        atomicMin(&ps.best, ((unsigned long long)__float_as_uint(est) << 32) |
+                                (unsigned)((n8 << 20) | (n4 << 10) | n2));
+      }
+    }
+    __syncthreads();
+    plan = (int)(unsigned)ps.best;
+  }
+  const int n8 = min(plan >> 20, B), n4 = min((plan >> 10) & 1023, B - n8),
+            n2 = min(plan & 1023, B - n8 - n4);
+  auto tier_of = [&](int rank) {
+    return rank < n8 ? 0 : (rank < n8 + n4 ? 1 : (rank < n8 + n4 + n2 ? 2 : 3));
+  };
+  auto us_of = [&](int rank) { return tt.us[tier_of(rank)] * (float)ps.len[ps.order[rank]]; };
+  // The workgroups of the ranks that run longer come first.
+  for (int r = tid; r < B; r += nt) {
+    const float us = us_of(r);
+    int first = 0;
+    for (int o = 0; o < B; ++o) {
+      const float u = us_of(o);
+      if (u > us || (u == us && o < r)) first += kTierParts[tier_of(o)] * H;
+    }
+    const int i = (int)blockIdx.x - first;
+    if (i >= 0 && i < kTierParts[tier_of(r)] * H) {
+      ps.row = ps.order[r];
+      ps.tier = tier_of(r);
+      ps.first = first;
+    }
+  }
+  __syncthreads();
+  const int b = __builtin_amdgcn_readfirstlane(ps.row);
+  const int tier = __builtin_amdgcn_readfirstlane(ps.tier);
+  const int i = (int)blockIdx.x - __builtin_amdgcn_readfirstlane(ps.first);
+  const int len = b >= 0 ? __builtin_amdgcn_readfirstlane(ps.len[b]) : 0;
+  __syncthreads();  // the scratch is the stages' from here on
+  if (b < 0) return;
+  Lds& lds = *reinterpret_cast<Lds*>(smem);
+  if (tier == 0)
+    prefill_tile16<Tag, Gates, 8, true>(pool, slot_idx, q, k, v, gates, y, H, G, heads_per_group,
+                                        T, b, i >> 3, i & 7, len, lds.l8);
+  else if (tier == 1)
+    prefill_tile16<Tag, Gates, 4, true>(pool, slot_idx, q, k, v, gates, y, H, G, heads_per_group,
+                                        T, b, i >> 2, i & 3, len, lds.l4);
+  else if (tier == 2)
+    prefill_tile16<Tag, Gates, 1, true>(pool, slot_idx, q, k, v, gates, y, H, G, heads_per_group,
+                                        T, b, i >> 1, i & 1, len, lds.l1);
+  else
+    prefill_tile16<Tag, Gates, 2, true>(pool, slot_idx, q, k, v, gates, y, H, G, heads_per_group,
+                                        T, b, i, 0, len, lds.l2);
+}
+
+// Ragged batches on an fp32 pool, of up to four tiles per CU: the rows' live lengths decide
 // the layout. Every workgroup derives the same plan from seq_lens:
 //   * rows ranked by live length, longest first (ties by row index);
 //   * three tiers by rank: the first n4 rows run in the quarter layout (four
@@ -876,12 +1060,10 @@ gdn_prefill_kernel(typename Storage<Tag>::T* __restrict__ pool,
 // A row's tiles compute the same bits in any layout.
 constexpr float kSplitCost = 0.745f;
 constexpr float kQuarterCost = 0.47f;
-constexpr int kMaxPlanRows = 1024;
 
-template <class Tag, class Gates>
+template <class Gates>
 __global__ void __launch_bounds__(256)
-gdn_prefill_planned_kernel(typename Storage<Tag>::T* __restrict__ pool,
-                           const int* __restrict__ slot_idx,
+gdn_prefill_planned_kernel(float* __restrict__ pool, const int* __restrict__ slot_idx,
                            const float* __restrict__ q, const float* __restrict__ k,
                            const float* __restrict__ v, Gates gates, float* __restrict__ y,
                            int B, int H, int G, int heads_per_group, int T, int cus,
@@ -954,7 +1136,7 @@ gdn_prefill_planned_kernel(typename Storage<Tag>::T* __restrict__ pool,
   if (i < 8 * n8 * H) {
     const int rank = i / (8 * H), rem = i - rank * 8 * H;
     const int b = order[rank];
-    prefill_tile<Tag, Gates, 8, true>(pool, slot_idx, q, k, v, gates, y, H, G, heads_per_group, T,
+    prefill_tile<Gates, 8, true>(pool, slot_idx, q, k, v, gates, y, H, G, heads_per_group, T,
                                       b, rem >> 3, rem & 7, lens[b], st);
     return;
   }
@@ -962,7 +1144,7 @@ gdn_prefill_planned_kernel(typename Storage<Tag>::T* __restrict__ pool,
   if (i < 4 * n4 * H) {
     const int rank = n8 + i / (4 * H), rem = i - (rank - n8) * 4 * H;
     const int b = order[rank];
-    prefill_tile<Tag, Gates, 4, true>(pool, slot_idx, q, k, v, gates, y, H, G, heads_per_group, T,
+    prefill_tile<Gates, 4, true>(pool, slot_idx, q, k, v, gates, y, H, G, heads_per_group, T,
                                       b, rem >> 2, rem & 3, lens[b], st);
     return;
   }
@@ -970,7 +1152,7 @@ gdn_prefill_planned_kernel(typename Storage<Tag>::T* __restrict__ pool,
   if (i < 2 * n2 * H) {
     const int rank = n8 + n4 + i / (2 * H), rem = i - (rank - n8 - n4) * 2 * H;
     const int b = order[rank];
-    prefill_tile<Tag, Gates, 1>(pool, slot_idx, q, k, v, gates, y, H, G, heads_per_group, T, b,
+    prefill_tile<Gates, 1>(pool, slot_idx, q, k, v, gates, y, H, G, heads_per_group, T, b,
                                 rem >> 1, rem & 1, lens[b], st);
     return;
   }
@@ -978,7 +1160,7 @@ gdn_prefill_planned_kernel(typename Storage<Tag>::T* __restrict__ pool,
   if (i < (B - n8 - n4 - n2) * H) {
     const int rank = n8 + n4 + n2 + i / H;
     const int b = order[rank];
-    prefill_tile<Tag, Gates, 2>(pool, slot_idx, q, k, v, gates, y, H, G, heads_per_group, T, b,
+    prefill_tile<Gates, 2>(pool, slot_idx, q, k, v, gates, y, H, G, heads_per_group, T, b,
                                 i - (i / H) * H, 0, lens[b], st);
   }
 }
@@ -1045,14 +1227,16 @@ void launch_decode_as(void* pool, const int32_t* slot_idx, int B, int H, int G, 
   const long n_wg = (long)B * H * P;
   const dim3 grid((unsigned)n_wg), block(tile_threads(kDecodeCols));
   const DeviceTopo topo = device_topo();
+  constexpr size_t kLds = sizeof(typename DecodeLds<Tag>::Tile) +
+                          kWaves * sizeof(typename DecodeLds<Tag>::QKWave);
   const StreamShape shape =
       stream_shape(n_wg, topo, !std::is_same<Tag, F32>::value,
-                   sizeof(TileLds) + kWaves * sizeof(QKLds),
+                   kLds,
                    launch_knob(BRAID_KNOB_DECODE_XCD_REMAP),
                    launch_knob(BRAID_KNOB_DECODE_WGS_PER_CU));
   // A launch capped at two resident workgroups per CU (its LDS request) takes
   // the two-waves-per-SIMD register budget.
-  const size_t lds_per_wg = shape.lds_pad + sizeof(TileLds) + kWaves * sizeof(QKLds);
+  const size_t lds_per_wg = shape.lds_pad + kLds;
   if constexpr (P == 1 && !std::is_same<Tag, F32>::value) {
     if (shape.lds_pad > 0 && (size_t)topo.lds_per_cu / lds_per_wg <= 2) {
       gdn_decode_kernel<Tag, Gates, P, 2><<<grid, block, shape.lds_pad, stream>>>(
@@ -1106,7 +1290,8 @@ int launch_decode(void* pool, int pool_dtype, const int32_t* slot_idx, int B, in
   return st != BRAID_OK ? st : ok();
 }
 
-// Prefill layout of a launch:
+// Prefill layout of a launch on an fp32 pool (the figures below are from 16-bit
+// pools, which ran these kernels when the lines were drawn):
 //   8: the eighth layout (one column and 8 rows per lane, eight workgroups
 //      per tile), when that leaves no CU with a second workgroup;
 //   4: the quarter layout (one column and 16 rows per lane, four workgroups
@@ -1141,31 +1326,19 @@ int prefill_layout(int n_tiles, int B, int T, bool ragged, int cus) {
   return ragged && B <= kMaxPlanRows && cus > 0 && n_tiles <= 4 * cus ? 0 : 2;
 }
 
+// fp32 pools.
 template <class Gates, int Layout>
-void launch_prefill_cols(void* pool, int pool_dtype, const int32_t* slot_idx, int B, int T,
-                         int H, int G, const float* q, const float* k, const float* v,
-                         Gates gates, float* y, hipStream_t stream) {
+void launch_prefill_cols(void* pool, const int32_t* slot_idx, int B, int T, int H, int G,
+                         const float* q, const float* k, const float* v, Gates gates, float* y,
+                         hipStream_t stream) {
   using LM = typename ScanLayoutOf<Layout>::type;
   const dim3 grid((unsigned)B * (unsigned)H * LM::kParts), block(64 * LM::kWaves);
-  const int hpg = H / G;
-  switch (pool_dtype) {
-    case BRAID_F32:
-      gdn_prefill_kernel<F32, Gates, Layout><<<grid, block, 0, stream>>>(
-          static_cast<float*>(pool), slot_idx, q, k, v, gates, y, H, G, hpg, T);
-      break;
-    case BRAID_F16:
-      gdn_prefill_kernel<F16, Gates, Layout><<<grid, block, 0, stream>>>(
-          static_cast<uint16_t*>(pool), slot_idx, q, k, v, gates, y, H, G, hpg, T);
-      break;
-    default:
-      gdn_prefill_kernel<BF16, Gates, Layout><<<grid, block, 0, stream>>>(
-          static_cast<uint16_t*>(pool), slot_idx, q, k, v, gates, y, H, G, hpg, T);
-      break;
-  }
+  gdn_prefill_kernel<Gates, Layout><<<grid, block, 0, stream>>>(
+      static_cast<float*>(pool), slot_idx, q, k, v, gates, y, H, G, H / G, T);
 }
 
 template <class Gates>
-void launch_prefill_planned(void* pool, int pool_dtype, const int32_t* slot_idx, int B, int T,
+void launch_prefill_planned(void* pool, const int32_t* slot_idx, int B, int T,
                             int H, int G, const float* q, const float* k, const float* v,
                             Gates gates, float* y, int cus, int forced, hipStream_t stream) {
   // At most one extra workgroup per CU for split tiles; the grid has room for
@@ -1180,24 +1353,9 @@ void launch_prefill_planned(void* pool, int pool_dtype, const int32_t* slot_idx,
     n_wg = std::max(n_wg, (8 * n8 + 4 * n4 + 2 * n2 + (B - n8 - n4 - n2)) * H);
   }
   const dim3 grid((unsigned)n_wg), block(256);
-  const int hpg = H / G;
-  switch (pool_dtype) {
-    case BRAID_F32:
-      gdn_prefill_planned_kernel<F32, Gates><<<grid, block, 0, stream>>>(
-          static_cast<float*>(pool), slot_idx, q, k, v, gates, y, B, H, G, hpg, T, cus,
-          max_extra, forced);
-      break;
-    case BRAID_F16:
-      gdn_prefill_planned_kernel<F16, Gates><<<grid, block, 0, stream>>>(
-          static_cast<uint16_t*>(pool), slot_idx, q, k, v, gates, y, B, H, G, hpg, T, cus,
-          max_extra, forced);
-      break;
-    default:
-      gdn_prefill_planned_kernel<BF16, Gates><<<grid, block, 0, stream>>>(
-          static_cast<uint16_t*>(pool), slot_idx, q, k, v, gates, y, B, H, G, hpg, T, cus,
-          max_extra, forced);
-      break;
-  }
+  gdn_prefill_planned_kernel<Gates><<<grid, block, 0, stream>>>(
+      static_cast<float*>(pool), slot_idx, q, k, v, gates, y, B, H, G, H / G, T, cus, max_extra,
+      forced);
 }
 
 // Host plan of a ragged prefill (the planned kernel's tiers), from the live
@@ -1336,7 +1494,10 @@ int simulate_prefill_plans(const std::vector<int>& lens, int H, int cus);
 // it has not seen lately instead of all of them at once.
 constexpr size_t kPlanCacheMax = 4096;
 
-int host_prefill_plan(const std::vector<int32_t>& seq_lens, int T, int H, int cus) {
+int simulate_prefill16_plans(const std::vector<int>& lens, int H, int cus, const TierTimes& tt);
+
+int host_prefill_plan(const std::vector<int32_t>& seq_lens, int T, int H, int cus,
+                      int pool_dtype = BRAID_F32) {
   std::vector<int> lens(seq_lens.size());
   for (size_t r = 0; r < lens.size(); ++r) lens[r] = std::min(std::max((int)seq_lens[r], 0), T);
   std::sort(lens.begin(), lens.end(), std::greater<int>());
@@ -1346,12 +1507,16 @@ int host_prefill_plan(const std::vector<int32_t>& seq_lens, int T, int H, int cu
   std::vector<int> key(lens);
   key.push_back(H);
   key.push_back(cus);
+  key.push_back(pool_dtype);
   {
     std::lock_guard<std::mutex> lock(mu);
     const auto it = cache.find(key);
     if (it != cache.end()) return it->second;
   }
-  const int plan = simulate_prefill_plans(lens, H, cus);
+  const int plan =
+      pool_dtype == BRAID_F32   ? simulate_prefill_plans(lens, H, cus)
+      : pool_dtype == BRAID_F16 ? simulate_prefill16_plans(lens, H, cus, tier_times<F16>())
+                                : simulate_prefill16_plans(lens, H, cus, tier_times<BF16>());
   std::lock_guard<std::mutex> lock(mu);
   const auto ins = cache.emplace(std::move(key), plan);
   if (ins.second) {  // another thread may have planned the same lengths meanwhile
@@ -1396,11 +1561,124 @@ int simulate_prefill_plans(const std::vector<int>& lens, int H, int cus) {
   return plan;
 }
 
+// The same choice for gdn_prefill16_planned_kernel: one workgroup per CU, in
+// the order of their durations, each on the CU that is free first. Ties: the
+// first plan found, fewer upgraded rows.
+int simulate_prefill16_plans(const std::vector<int>& lens, int H, int cus, const TierTimes& tt) {
+  const int B = (int)lens.size();
+  float best = INFINITY;
+  int plan = 0;
+  std::vector<std::pair<float, long>> jobs;  // duration, workgroups
+  for (int n8 = 0; n8 <= std::min(B, kMaxN8); ++n8)
+    for (int n4 = 0; n4 <= std::min(B - n8, kMaxN4); ++n4)
+      for (int n2 = 0; n2 <= std::min(B - n8 - n4, kMaxN2); ++n2) {
+        jobs.clear();
+        double work = 0.0;
+        for (int r = 0; r < B; ++r) {
+          const int t = r < n8 ? 0 : (r < n8 + n4 ? 1 : (r < n8 + n4 + n2 ? 2 : 3));
+          if (lens[r] <= 0) continue;
+          const float us = tt.us[t] * (float)lens[r];
+          const long n = (long)kTierParts[t] * H;
+          jobs.emplace_back(us, n);
+          work += (double)us * n;
+        }
+        if (jobs.empty()) continue;
+        std::sort(jobs.begin(), jobs.end(), std::greater<std::pair<float, long>>());
+        if (std::max(jobs[0].first, (float)(work / cus)) >= best) continue;
+        std::map<float, long> free_at;  // CUs by the time they are free
+        free_at[0.f] = cus;
+        float end = 0.f;
+        for (auto [us, n] : jobs)
+          while (n > 0) {
+            const auto it = free_at.begin();
+            const long m = std::min(n, it->second);
+            const float t = it->first + us;
+            if (m == it->second) free_at.erase(it);
+            else it->second -= m;
+            free_at[t] += m;
+            end = std::max(end, t);
+            n -= m;
+          }
+        if (end < best) {
+          best = end;
+          plan = (n8 << 20) | (n4 << 10) | n2;
+        }
+      }
+  return plan;
+}
+
+// Prefill layout of a launch on a 16-bit pool: the most workgroups per tile
+// that leave no CU with a second one (a token's time, one workgroup per CU:
+// eighth 0.160 us, quarter 0.172, split 0.250, whole 0.392, fp16), planned per
+// row for ragged batches of up to four tiles per CU, whole otherwise. The
+// PREFILL_LAYOUT launch knob overrides the choice.
+int prefill_layout16(int n_tiles, int B, bool ragged, int cus) {
+  const int forced = launch_knob(BRAID_KNOB_PREFILL_LAYOUT);
+  if (forced == 1 || forced == 2 || forced == 4 || forced == 8) return forced;
+  if (forced == 0 && ragged && B <= kMaxPlanRows) return 0;
+  if (cus > 0 && 8 * n_tiles <= cus) return 8;
+  if (ragged && B > 1 && B <= kMaxPlanRows && cus > 0 && n_tiles <= 4 * cus) return 0;
+  if (cus > 0 && 4 * n_tiles <= cus) return 4;
+  if (cus > 0 && 2 * n_tiles <= cus) return 1;
+  return 2;
+}
+
+template <class Tag, class Gates>
+void launch_prefill16(void* pool, int pool_dtype, const int32_t* slot_idx, int B, int T, int H,
+                      int G, const float* q, const float* k, const float* v, Gates gates, float* y,
+                      const std::vector<int32_t>* host_lens, int plan_hint, hipStream_t stream) {
+  const int cus = device_cus();
+  uint16_t* const p = static_cast<uint16_t*>(pool);
+  const int layout = prefill_layout16(B * H, B, gates.ragged(), cus);
+  auto run = [&](auto kern, int parts, int threads) {
+    kern<<<dim3((unsigned)B * (unsigned)H * (unsigned)parts), dim3(threads), 0, stream>>>(
+        p, slot_idx, q, k, v, gates, y, H, G, H / G, T);
+  };
+  auto run_layout = [&](int l) {
+    if (l == 8) run(gdn_prefill16_kernel<Tag, Gates, 8>, 8, Scan16Map<8>::kThreads);
+    else if (l == 4) run(gdn_prefill16_kernel<Tag, Gates, 4>, 4, Scan16Map<4>::kThreads);
+    else if (l == 1) run(gdn_prefill16_kernel<Tag, Gates, 1>, 2, Scan16Map<1>::kThreads);
+    else run(gdn_prefill16_kernel<Tag, Gates, 2>, 1, Scan16Map<2>::kThreads);
+  };
+  if (layout != 0) return run_layout(layout);
+  // The PREFILL_PLAN knob (measurement), else the host's plan from lengths it
+  // can read, else the caller's, else the kernel's own (-1).
+  const int some_cus = cus > 0 ? cus : 256;
+  int plan = launch_knob(BRAID_KNOB_PREFILL_PLAN);
+  const bool chosen = plan < 0 && launch_knob(BRAID_KNOB_PREFILL_LAYOUT) < 0;
+  if (chosen) plan = host_lens != nullptr
+                         ? host_prefill_plan(*host_lens, T, H, some_cus, pool_dtype)
+                         : plan_hint;
+  int max_extra = std::min(some_cus, 7 * B * H), n_wg = B * H + max_extra;
+  if (plan >= 0) {
+    const int n8 = std::min(plan >> 20, B), n4 = std::min((plan >> 10) & 1023, B - n8);
+    const int n2 = std::min(plan & 1023, B - n8 - n4);
+    plan = (n8 << 20) | (n4 << 10) | n2;
+    // One tier: its own kernel.
+    if (chosen && (n8 == B || n4 == B || n2 == B || plan == 0))
+      return run_layout(n8 == B ? 8 : (n4 == B ? 4 : (n2 == B ? 1 : 2)));
+    n_wg = (B + 7 * n8 + 3 * n4 + n2) * H;
+  }
+  gdn_prefill16_planned_kernel<Tag, Gates>
+      <<<dim3((unsigned)n_wg), dim3(Scan16Map<2>::kThreads), 0, stream>>>(
+          p, slot_idx, q, k, v, gates, y, B, H, G, H / G, T, some_cus, max_extra, plan);
+}
+
 template <class Gates>
 int launch_prefill(void* pool, int pool_dtype, const int32_t* slot_idx, int B, int T, int H,
                    int G, const float* q, const float* k, const float* v, Gates gates,
                    float* y, const std::vector<int32_t>* host_lens, hipStream_t stream,
                    int plan_hint = -1) {
+  if (pool_dtype != BRAID_F32) {
+    if (pool_dtype == BRAID_F16)
+      launch_prefill16<F16>(pool, pool_dtype, slot_idx, B, T, H, G, q, k, v, gates, y, host_lens,
+                            plan_hint, stream);
+    else
+      launch_prefill16<BF16>(pool, pool_dtype, slot_idx, B, T, H, G, q, k, v, gates, y, host_lens,
+                             plan_hint, stream);
+    const int st = hip_status(hipGetLastError(), "launching gdn_prefill16_kernel");
+    return st != BRAID_OK ? st : ok();
+  }
   const int cus = device_cus();
   int layout = prefill_layout(B * H, B, T, gates.ragged(), cus);
   // With the live lengths on the host, every ragged batch the planned kernel
@@ -1427,23 +1705,19 @@ int launch_prefill(void* pool, int pool_dtype, const int32_t* slot_idx, int B, i
     layout = n8 == B ? 8 : (n4 == B ? 4 : (n2 == B ? 1 : 0));
   }
   if (layout == 8)
-    launch_prefill_cols<Gates, 8>(pool, pool_dtype, slot_idx, B, T, H, G, q, k, v, gates, y,
-                                  stream);
+    launch_prefill_cols<Gates, 8>(pool, slot_idx, B, T, H, G, q, k, v, gates, y, stream);
   else if (layout == 4)
-    launch_prefill_cols<Gates, 4>(pool, pool_dtype, slot_idx, B, T, H, G, q, k, v, gates, y,
-                                  stream);
+    launch_prefill_cols<Gates, 4>(pool, slot_idx, B, T, H, G, q, k, v, gates, y, stream);
   else if (layout == 1)
-    launch_prefill_cols<Gates, 1>(pool, pool_dtype, slot_idx, B, T, H, G, q, k, v, gates, y,
-                                  stream);
+    launch_prefill_cols<Gates, 1>(pool, slot_idx, B, T, H, G, q, k, v, gates, y, stream);
   else if (layout == 2)
-    launch_prefill_cols<Gates, 2>(pool, pool_dtype, slot_idx, B, T, H, G, q, k, v, gates, y,
-                                  stream);
+    launch_prefill_cols<Gates, 2>(pool, slot_idx, B, T, H, G, q, k, v, gates, y, stream);
   else {
     // The PREFILL_PLAN knob (measurement) forces a plan; otherwise an eager
     // call runs the host's plan and a captured one leaves it to the kernel.
     int forced = launch_knob(BRAID_KNOB_PREFILL_PLAN);
     if (forced < 0) forced = host_plan;
-    launch_prefill_planned<Gates>(pool, pool_dtype, slot_idx, B, T, H, G, q, k, v, gates, y,
+    launch_prefill_planned<Gates>(pool, slot_idx, B, T, H, G, q, k, v, gates, y,
                                   cus > 0 ? cus : 256, forced, stream);
   }
   const int st = hip_status(hipGetLastError(), "launching gdn_prefill_kernel");
@@ -1696,6 +1970,17 @@ extern "C" int braid_gdn_conv_decode_raw(void* pool, int pool_dtype, int64_t n_s
                             A, dt_bias, nullptr});
   return go(RawGates<BF16>{static_cast<const uint16_t*>(a_raw),
                            static_cast<const uint16_t*>(b_raw), A, dt_bias, nullptr});
+}
+
+extern "C" int braid_prefill_plan_pool(const int32_t* seq_lens_host, int B, int T, int H, int cus,
+                                      int pool_dtype) {
+  if (pool_dtype != BRAID_F32 && pool_dtype != BRAID_F16 && pool_dtype != BRAID_BF16)
+    return -fail(BRAID_EINVAL, "state pool must be fp32, fp16 or bf16");
+  if (seq_lens_host == nullptr || B <= 0 || T < 0 || H <= 0 || cus <= 0)
+    return -fail(BRAID_EINVAL,
+                 "braid_prefill_plan_pool needs host lengths, B > 0, T >= 0, H > 0, cus > 0");
+  return host_prefill_plan(std::vector<int32_t>(seq_lens_host, seq_lens_host + B), T, H, cus,
+                           pool_dtype);
 }
 
 extern "C" int braid_prefill_plan(const int32_t* seq_lens_host, int B, int T, int H, int cus) {

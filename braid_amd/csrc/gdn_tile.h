@@ -24,11 +24,14 @@
 //      (w0 + w1) + (w2 + w3), evaluated the same way by every lane that needs
 //      the total.
 //
-// Prefill layouts (ScanMap: 2 columns per lane, or 1 for small launches, whose
-// tiles are then split over two workgroups; ScanMapQuarter: 1 column and 16
-// rows per lane, a tile over four workgroups): the same rows, chains and tree.
-// A column's arithmetic does not depend on which lane holds it, so the results
-// are the decode layout's bits.
+// The reductions above are the fp32 pool's. A 16-bit pool's decode holds its tile
+// in the same lanes but takes its sums on the matrix cores (gdn_mfma.h).
+//
+// Prefill layouts of an fp32 pool (ScanMap: 2 columns per lane, or 1 for small
+// launches, whose tiles are then split over two workgroups; ScanMapQuarter: 1
+// column and 16 rows per lane, a tile over four workgroups): the same rows,
+// chains and tree. A column's arithmetic does not depend on which lane holds
+// it, so the results are the decode layout's bits. (16-bit pools: gdn_scan16.h.)
 //
 // The state lives in registers in its STORAGE type. Each token widens it to
 // fp32, runs the recurrence in fp32 and narrows it back, exactly as a decode
@@ -193,20 +196,6 @@ struct Row<BF16, N> : RowHalf<N> {
   }
 };
 
-// One column per lane (the split prefill layout). The 16-bit rows keep their
-// element in the low half of a 32-bit register and narrow through the same
-// packed conversion as the pairs (the high half is discarded), so the
-// rounding is the pairs' bit for bit and the compiler cannot fuse it into the
-// producing fma.
-template <>
-struct Row<F32, 1> {
-  float d;
-  __device__ __forceinline__ void load_nt(const float* p) { d = __builtin_nontemporal_load(p); }
-  __device__ __forceinline__ void store_nt(float* p) const { __builtin_nontemporal_store(d, p); }
-  __device__ __forceinline__ float get(int) const { return d; }
-  __device__ __forceinline__ void set1(float x) { d = x; }
-};
-
 // x as an opaque fp32 register value: a narrowing of the result then starts
 // from the rounded fp32 value. Without it the backend can fuse the producing
 // fma with a single-element fp16 narrowing into one mixed-precision fma that
@@ -217,46 +206,8 @@ __device__ __forceinline__ float opaque(float x) {
   return x;
 }
 
-// The first term of a kv chain, S * kh, as fma(S, kh, -0): equal to the
-// rounded product for every input (adding -0 changes no value and keeps a -0
-// product), and one mixed-precision fma on a 16-bit S instead of a widening
-// and a multiply. The -0 goes through opaque() so the fma is not folded back
-// into the multiply.
-__device__ __forceinline__ float first_term(float s, float kh, float neg_zero) {
-  return fmaf(s, kh, neg_zero);
-}
-
-struct RowHalf1 {
-  uint32_t raw;  // the element in bits 0..15
-  __device__ __forceinline__ void load_nt(const uint16_t* p) {
-    raw = __builtin_nontemporal_load(p);
-  }
-  __device__ __forceinline__ void store_nt(uint16_t* p) const {
-    __builtin_nontemporal_store((uint16_t)raw, p);
-  }
-  __device__ __forceinline__ uint32_t bits(int) const { return raw & 0xffffu; }
-};
-
-template <>
-struct Row<F16, 1> : RowHalf1 {
-  __device__ __forceinline__ float get(int c) const { return f16_widen(bits(c)); }
-  __device__ __forceinline__ void set1(float x) { raw = pack_f16x2(x, 0.f) & 0xffffu; }
-};
-
-template <>
-struct Row<BF16, 1> : RowHalf1 {
-  __device__ __forceinline__ float get(int c) const { return bf16_widen(bits(c)); }
-  __device__ __forceinline__ void set1(float x) { raw = pack_bf16x2(x, 0.f) & 0xffffu; }
-};
-
-// Two rows' elements of one column (the one-column prefill layouts): row a in
-// bits 0..15 of one register, row b in bits 16..31, so one packed conversion
-// narrows both (the mixed-precision fma reads either half directly). Each
-// element is rounded on its own, as the single-element rows round it.
-template <class Tag>
-struct RowPair1;
-template <>
-struct RowPair1<F32> {
+// Two rows' elements of one column (the one-column prefill layouts).
+struct RowPair1 {
   float d0, d1;
   __device__ __forceinline__ void load_nt(const float* a, const float* b) {
     d0 = __builtin_nontemporal_load(a);
@@ -271,27 +222,6 @@ struct RowPair1<F32> {
     d0 = lo;
     d1 = hi;
   }
-};
-struct RowHalfPair {
-  uint32_t raw;
-  __device__ __forceinline__ void load_nt(const uint16_t* a, const uint16_t* b) {
-    raw = (uint32_t)__builtin_nontemporal_load(a) | ((uint32_t)__builtin_nontemporal_load(b) << 16);
-  }
-  __device__ __forceinline__ void store_nt(uint16_t* a, uint16_t* b) const {
-    __builtin_nontemporal_store((uint16_t)raw, a);
-    __builtin_nontemporal_store((uint16_t)(raw >> 16), b);
-  }
-  __device__ __forceinline__ uint32_t bits(int h) const { return h ? raw >> 16 : raw & 0xffffu; }
-};
-template <>
-struct RowPair1<F16> : RowHalfPair {
-  __device__ __forceinline__ float get(int h) const { return f16_widen(bits(h)); }
-  __device__ __forceinline__ void set(float lo, float hi) { raw = pack_f16x2(lo, hi); }
-};
-template <>
-struct RowPair1<BF16> : RowHalfPair {
-  __device__ __forceinline__ float get(int h) const { return bf16_widen(bits(h)); }
-  __device__ __forceinline__ void set(float lo, float hi) { raw = pack_bf16x2(lo, hi); }
 };
 
 // N consecutive floats from / to 16-byte-aligned memory (global or LDS).
@@ -1015,20 +945,17 @@ __device__ __forceinline__ void gdn_token(const LaneMap<CPL, kSplit>& L,
 // w * 32 + rg + 4 i), in the scan layout: the decode token's arithmetic, each
 // element's operations in the decode's order. kh / qh hold the row block's 32
 // normalised key / query entries in row order.
-// kOpaqueNarrow: narrow each new state element through opaque() (for callers
-// whose code shape lets the backend contract the narrowing).
-template <class Tag, int CPL, bool kOpaqueNarrow = false>
-__device__ __forceinline__ void scan_token(Row<Tag, CPL> (&S)[kRowGroups][kRowsPerLane],
+template <int CPL>
+__device__ __forceinline__ void scan_token(Row<F32, CPL> (&S)[kRowGroups][kRowsPerLane],
                                            const float (&kh)[kRowsPerWave],
                                            const float (&qh)[kRowsPerWave],
                                            const float (&v)[CPL], float alpha, float beta,
                                            float (&y)[CPL]) {
   float ch[kRowGroups][CPL];
-  const float nz = opaque(-0.0f);
 #pragma unroll
   for (int rg = 0; rg < kRowGroups; ++rg) {
 #pragma unroll
-    for (int c = 0; c < CPL; ++c) ch[rg][c] = first_term(S[rg][0].get(c), kh[rg], nz);
+    for (int c = 0; c < CPL; ++c) ch[rg][c] = S[rg][0].get(c) * kh[rg];
 #pragma unroll
     for (int i = 1; i < kRowsPerLane; ++i) {
 #pragma unroll
@@ -1048,22 +975,13 @@ __device__ __forceinline__ void scan_token(Row<Tag, CPL> (&S)[kRowGroups][kRowsP
 #pragma unroll
     for (int i = 0; i < kRowsPerLane; ++i) {
       const int r = rg + kRowGroups * i;
-      if constexpr (CPL == 1) {
-        // Both uses of the new value take the barrier's output, so it costs
-        // no register copy.
-        float n0 = fmaf(alpha, S[rg][i].get(0), kh[r] * delta[0]);
-        if constexpr (kOpaqueNarrow) n0 = opaque(n0);
-        S[rg][i].set1(n0);
-        ch[rg][0] = fmaf(n0, qh[r], ch[rg][0]);
-      } else {
 #pragma unroll
-        for (int c = 0; c < CPL; c += 2) {
-          const float n0 = fmaf(alpha, S[rg][i].get(c), kh[r] * delta[c]);
-          const float n1 = fmaf(alpha, S[rg][i].get(c + 1), kh[r] * delta[c + 1]);
-          S[rg][i].set2(c, n0, n1);
-          ch[rg][c] = fmaf(n0, qh[r], ch[rg][c]);
-          ch[rg][c + 1] = fmaf(n1, qh[r], ch[rg][c + 1]);
-        }
+      for (int c = 0; c < CPL; c += 2) {
+        const float n0 = fmaf(alpha, S[rg][i].get(c), kh[r] * delta[c]);
+        const float n1 = fmaf(alpha, S[rg][i].get(c + 1), kh[r] * delta[c + 1]);
+        S[rg][i].set2(c, n0, n1);
+        ch[rg][c] = fmaf(n0, qh[r], ch[rg][c]);
+        ch[rg][c + 1] = fmaf(n1, qh[r], ch[rg][c + 1]);
       }
     }
   }
@@ -1075,16 +993,14 @@ __device__ __forceinline__ void scan_token(Row<Tag, CPL> (&S)[kRowGroups][kRowsP
 // The one-column layout's token over row pairs: P[p][i] holds rows of row
 // groups 2p (low half) and 2p + 1 (high half), i.e. rows w * 32 + rg + 4 i.
 // Each element's operations and each chain's order are scan_token's.
-template <class Tag, bool kOpaqueNarrow = false>
-__device__ __forceinline__ void scan_token_pairs(RowPair1<Tag> (&P)[2][kRowsPerLane],
+__device__ __forceinline__ void scan_token_pairs(RowPair1 (&P)[2][kRowsPerLane],
                                                  const float (&kh)[kRowsPerWave],
                                                  const float (&qh)[kRowsPerWave], float v,
                                                  float alpha, float beta, float& y) {
   float ch[kRowGroups];
-  const float nz = opaque(-0.0f);
 #pragma unroll
   for (int rg = 0; rg < kRowGroups; ++rg) {
-    ch[rg] = first_term(P[rg >> 1][0].get(rg & 1), kh[rg], nz);
+    ch[rg] = P[rg >> 1][0].get(rg & 1) * kh[rg];
 #pragma unroll
     for (int i = 1; i < kRowsPerLane; ++i)
       ch[rg] = fmaf(P[rg >> 1][i].get(rg & 1), kh[rg + kRowGroups * i], ch[rg]);
@@ -1101,7 +1017,6 @@ __device__ __forceinline__ void scan_token_pairs(RowPair1<Tag> (&P)[2][kRowsPerL
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         n[h] = fmaf(alpha, P[p][i].get(h), kh[2 * p + h + kRowGroups * i] * delta);
-        if constexpr (kOpaqueNarrow) n[h] = opaque(n[h]);
       }
       P[p][i].set(n[0], n[1]);
 #pragma unroll
@@ -1116,16 +1031,14 @@ __device__ __forceinline__ void scan_token_pairs(RowPair1<Tag> (&P)[2][kRowsPerL
 // is row w * 32 + 2 rgh + rgl + 4 i, kh / qh hold the same rows. Each
 // element's operations are scan_token's (and so the decode's), in the same
 // order; the column totals follow the layout's tree.
-template <class Tag, bool kOpaqueNarrow = false>
-__device__ __forceinline__ void scan_token_quarter(RowPair1<Tag> (&P)[kRowsPerLane],
+__device__ __forceinline__ void scan_token_quarter(RowPair1 (&P)[kRowsPerLane],
                                                    const float (&kh)[2][kRowsPerLane],
                                                    const float (&qh)[2][kRowsPerLane], float v,
                                                    float alpha, float beta, float& y) {
   float ch[2];
-  const float nz = opaque(-0.0f);
 #pragma unroll
   for (int g = 0; g < 2; ++g) {
-    ch[g] = first_term(P[0].get(g), kh[g][0], nz);
+    ch[g] = P[0].get(g) * kh[g][0];
 #pragma unroll
     for (int i = 1; i < kRowsPerLane; ++i) ch[g] = fmaf(P[i].get(g), kh[g][i], ch[g]);
   }
@@ -1138,7 +1051,6 @@ __device__ __forceinline__ void scan_token_quarter(RowPair1<Tag> (&P)[kRowsPerLa
 #pragma unroll
     for (int g = 0; g < 2; ++g) {
       n[g] = fmaf(alpha, P[i].get(g), kh[g][i] * delta);
-      if constexpr (kOpaqueNarrow) n[g] = opaque(n[g]);
     }
     P[i].set(n[0], n[1]);
 #pragma unroll
@@ -1152,13 +1064,11 @@ __device__ __forceinline__ void scan_token_quarter(RowPair1<Tag> (&P)[kRowsPerLa
 // (row w * 32 + rg + 4 i); kh / qh hold the same rows. Each element's
 // operations are scan_token's (and so the decode's), in the same order; the
 // column totals follow the layout's tree.
-template <class Tag, bool kOpaqueNarrow = false>
-__device__ __forceinline__ void scan_token_eighth(RowPair1<Tag> (&P)[kRowsPerLane / 2],
+__device__ __forceinline__ void scan_token_eighth(RowPair1 (&P)[kRowsPerLane / 2],
                                                   const float (&kh)[kRowsPerLane],
                                                   const float (&qh)[kRowsPerLane], float v,
                                                   float alpha, float beta, float& y) {
-  const float nz = opaque(-0.0f);
-  float ch = first_term(P[0].get(0), kh[0], nz);
+  float ch = P[0].get(0) * kh[0];
 #pragma unroll
   for (int i = 1; i < kRowsPerLane; ++i) ch = fmaf(P[i >> 1].get(i & 1), kh[i], ch);
   const float kv = add_xor8(add_xor4(add_xor2(add_xor1(ch))));
@@ -1170,7 +1080,6 @@ __device__ __forceinline__ void scan_token_eighth(RowPair1<Tag> (&P)[kRowsPerLan
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       n[h] = fmaf(alpha, P[m].get(h), kh[2 * m + h] * delta);
-      if constexpr (kOpaqueNarrow) n[h] = opaque(n[h]);
     }
     P[m].set(n[0], n[1]);
 #pragma unroll
@@ -1179,20 +1088,20 @@ __device__ __forceinline__ void scan_token_eighth(RowPair1<Tag> (&P)[kRowsPerLan
   y = add_xor8(add_xor4(add_xor2(add_xor1(ch)))) * kYScale;
 }
 
-// Computes one token's gates once per tile and leaves them in lds.gate for
-// gdn_token: wave 0 evaluates alpha (exp, log1p, exp), wave 1 beta (exp and a
+// Computes one token's gates once per tile and leaves them in the tile's LDS
+// (gate) for the token: wave 0 evaluates alpha (exp, log1p, exp), wave 1 beta (exp and a
 // divide), from the inputs every wave loaded. The next workgroup barrier
 // publishes them. The
 // arithmetic is the policy's own, so which wave runs it changes no bit.
 template <class Gates, class LM>
 __device__ __forceinline__ void publish_gates(const LM& L, const Gates& gates, const GateRaw& r,
-                                              const GateConst& c, TileLds& lds) {
+                                              const GateConst& c, float (&gate)[2]) {
   if (L.wave == 0) {
     const float a = gates.alpha_of(r, c);
-    if (L.lane == 0) lds.gate[0] = a;
+    if (L.lane == 0) gate[0] = a;
   } else if (L.wave == 1) {
     const float bt = gates.eval_beta(r);
-    if (L.lane == 0) lds.gate[1] = bt;
+    if (L.lane == 0) gate[1] = bt;
   }
 }
 

@@ -54,6 +54,7 @@ SIGNATURES = {
     "braid_set_launch_override": ([_i32, _i32], _i32),
     "braid_get_launch_override": ([_i32], _i32),
     "braid_prefill_plan": ([_vp, _i32, _i32, _i32, _i32], _i32),
+    "braid_prefill_plan_pool": ([_vp, _i32, _i32, _i32, _i32, _i32], _i32),
     "braid_gdn_decode": ([_vp, _i32, _i64, _i32, _i32, _i32, _i32, _vp, _i32,
                           _vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _vp, _vp], _i32),
     "braid_gdn_decode_raw": ([_vp, _i32, _i64, _i32, _i32, _i32, _i32, _vp, _i32,
@@ -334,18 +335,20 @@ class GDNKernels:
             return
         _check(seq_lens is not None, "plan_lens plans a ragged batch: seq_lens is required")
         _check(len(plan_lens) == B, "plan_lens must have one entry per batch row")
-        plan = self.prefill_plan(plan_lens, T, H, pool.device)
+        plan = self.prefill_plan(plan_lens, T, H, pool.device, pool.dtype)
         self._call("braid_gdn_prefill_raw_plan", pool.device, _ptr(pool), pdt, pool.size(0), H,
                    G, SS, HD, _ptr(slot_idx), B, T, _ptr(q), _ptr(k), _ptr(v), _ptr(a_raw),
                    _ptr(b_raw), adt, _ptr(A), _ptr(dt_bias), _ptr(y), _ptr(seq_lens), plan)
 
-    def prefill_plan(self, lens: Sequence[int], T: int, H: int, device=None) -> int:
+    def prefill_plan(self, lens: Sequence[int], T: int, H: int, device=None,
+                     pool_dtype: torch.dtype = torch.float32) -> int:
         """The plan (n8 * 2^20 + n4 * 2^10 + n2) an eager ragged prefill of
-        these host lengths runs on ``device`` (braid_prefill_plan)."""
+        these host lengths runs on ``device`` with a pool of ``pool_dtype``
+        (braid_prefill_plan_pool)."""
         cus = torch.cuda.get_device_properties(device).multi_processor_count
         arr = (ctypes.c_int32 * len(lens))(*[int(x) for x in lens])
-        plan = self._lib.braid_prefill_plan(ctypes.cast(arr, ctypes.c_void_p), len(lens), T, H,
-                                            cus)
+        plan = self._lib.braid_prefill_plan_pool(ctypes.cast(arr, ctypes.c_void_p), len(lens), T,
+                                                 H, cus, _POOL_DTYPES[pool_dtype])
         _check(plan >= 0, self._lib.braid_last_error().decode())
         return plan
 

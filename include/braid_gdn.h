@@ -90,6 +90,13 @@ enum braid_launch_knob {
  * counterpart in the reference.
  */
 int braid_prefill_plan(const int32_t* seq_lens_host, int B, int T, int H, int cus);
+/*
+ * The same for a pool of pool_dtype: a 16-bit pool's tiers have other times
+ * (braid_prefill_plan is the fp32 pool's plan). Any plan suits any pool; this
+ * one is what an eager call on such a pool chooses.
+ */
+int braid_prefill_plan_pool(const int32_t* seq_lens_host, int B, int T, int H, int cus,
+                            int pool_dtype);
 
 /* Sets a knob (value < 0 clears it). BRAID_EINVAL for an unknown knob. */
 int braid_set_launch_override(int knob, int value);
