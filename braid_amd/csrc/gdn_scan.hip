@@ -24,6 +24,7 @@
 
 #include "capi_common.h"
 #include "conv_common.h"
+#include "gated_unit.h"
 #include "gdn_mfma.h"
 #include "gdn_scan16.h"
 #include "gdn_tile.h"
@@ -169,20 +170,80 @@ struct ConvDecodeLds {
   typename DecodeLds<Tag>::QKWave qk[std::is_same<Tag, F32>::value ? 1 : HPG * kWaves];
 };
 
+// Where a conv + decode workgroup's outputs go: y rows (PlainOut), or through
+// the gated RMSNorm readout (GatedOut): core, and one partial max of |core| per
+// (row, head) unit for the quantize pass that follows. The readout's unit is
+// the tile's 128 outputs, all of which are at hand when the token ends, so y
+// never goes to memory and the readout's own launch falls away.
+struct PlainOut {
+  float* y;
+  struct Pre {};
+  __device__ __forceinline__ void pin_args() const { braid::pin_args(y); }
+  __device__ __forceinline__ Pre load(size_t, int, int) const { return Pre{}; }
+};
+template <class ATag>
+struct GatedOut {
+  using AT = typename ATag::T;
+  const AT* z;
+  const float* gamma;
+  float eps;
+  AT* core;
+  float* partial;
+  // The lane's four gate values and gammas (lanes 0-31 of a tile's first wave;
+  // 32-63 hold the same ones), read with the tile and used after it.
+  struct Pre {
+    float z[4];
+    quant::f32x4 gamma;
+  };
+  __device__ __forceinline__ void pin_args() const { braid::pin_args(z, gamma, core, partial); }
+  __device__ __forceinline__ Pre load(size_t unit, int wave, int lane) const {
+    Pre p{};
+    if (wave == 0) {
+      const int c = 4 * (lane & 31);
+      quant::load4(ATag{}, z, (long)unit * kHD + c, p.z);
+      p.gamma = *reinterpret_cast<const quant::f32x4*>(gamma + c);
+    }
+    return p;
+  }
+  // The unit's readout from its outputs y (four per lane), on the first wave.
+  __device__ __forceinline__ void finish(const Pre& p, size_t unit, int lane, float (&y)[4]) const {
+    float m = 0.f;
+    quant::gated_unit<ATag>(y, p.z, p.gamma, eps, lane < 32, core, (long)unit * kHD + 4 * (lane & 31),
+                            m);
+    m = quant::nan_max(m, quant::lane_xor<1>(m));
+    m = quant::nan_max(m, quant::lane_xor<2>(m));
+    m = quant::nan_max(m, quant::lane_xor<4>(m));
+    m = quant::nan_max(m, quant::lane_xor<8>(m));
+    m = quant::nan_max(m, quant::lane_xor<16>(m));
+    if (lane == 0) partial[unit] = m;
+  }
+};
+
 // The decode token of tile t of a conv + decode workgroup, on the conv
 // outputs in LDS (after the barrier that publishes them), then the stores.
-template <class Tag, int HPG, class LM>
+// unit: the tile's (row, head) index.
+template <class Tag, int HPG, class LM, class Out>
 __device__ __forceinline__ void decode_token_from_lds(const LM& L,
                                                       Row<Tag, kDecodeCols> (&S)[kRowsPerLane],
                                                       ConvDecodeLds<Tag, HPG>& lds, int t,
                                                       typename Storage<Tag>::T* tile,
-                                                      float* y_row) {
+                                                      const Out& out, const typename Out::Pre& pre,
+                                                      size_t unit) {
   constexpr int CPL = kDecodeCols;
+  constexpr bool kGated = !std::is_same<Out, PlainOut>::value;
   float vv[CPL];
   load_cols(L, lds.qkv[2 + t], vv);
   auto store_state = [&] {
 #pragma unroll
     for (int i = 0; i < kRowsPerLane; ++i) store_row(S[i], L, tile + (size_t)L.row(i) * kHD);
+  };
+  // Column c's total over the four row blocks, for the readout's lanes.
+  auto totals4 = [&](float (*buf)[kHD], float (&o)[4]) {
+    float p[kWaves][4];
+#pragma unroll
+    for (int j = 0; j < kWaves; ++j) loadN<4>(&buf[j][4 * (L.lane & 31)], p[j]);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) o[c] = (p[0][c] + p[1][c]) + (p[2][c] + p[3][c]);
   };
   if constexpr (std::is_same<Tag, F32>::value) {
     QK qk;
@@ -190,7 +251,15 @@ __device__ __forceinline__ void decode_token_from_lds(const LM& L,
     float yy[CPL];
     gdn_token<Tag, CPL>(L, S, qk, vv, lds.tile[t], yy);
     store_state();
-    if (L.stores_y()) store_cols(L, y_row, yy);
+    if constexpr (!kGated) {
+      if (L.stores_y()) store_cols(L, out.y + unit * kHD, yy);
+    } else if (L.wave == 0) {
+      float y[4];
+      totals4(lds.tile[t].y, y);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) y[c] *= kYScale;
+      out.finish(pre, unit, L.lane, y);
+    }
   } else {
     float2 q2, k2;
     load_qk2(L, lds.qkv[0], lds.qkv[1], q2, k2);
@@ -199,22 +268,36 @@ __device__ __forceinline__ void decode_token_from_lds(const LM& L,
     float delta[CPL];
     gdn_token16<Tag, CPL>(L, S, qk, vv, lds.tile[t], delta);
     store_state();
-    token16_readout<Tag, CPL>(L, qk, lds.tile[t], delta, y_row);
+    if constexpr (!kGated) {
+      token16_readout<Tag, CPL>(L, qk, lds.tile[t], delta, out.y + unit * kHD);
+    } else if (L.wave == 0) {
+      float kv[4], sq[4], v[4], y[4];
+      totals4(lds.tile[t].kv, kv);
+      totals4(lds.tile[t].sq, sq);
+      loadN<4>(&lds.qkv[2 + t][4 * (L.lane & 31)], v);
+      const float alpha_s = lds.tile[t].gate[0] * (1.f / Parts<Tag>::kScale);
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+        y[c] = readout_of(alpha_s, sq[c], delta_of(v[c], alpha_s, lds.tile[t].gate[1], kv[c]),
+                          qk.kq);
+      out.finish(pre, unit, L.lane, y);
+    }
   }
 }
 
-template <class Tag, class XT, class Gates, int HPG>
+template <class Tag, class XT, class Gates, int HPG, class Out>
 __device__ __forceinline__ void conv_decode_body(typename Storage<Tag>::T* __restrict__ pool,
                                                  float* __restrict__ conv_pool,
                                                  const int* __restrict__ slot_idx,
                                                  const XT* __restrict__ x,
                                                  const float* __restrict__ conv_w,
                                                  const float* __restrict__ conv_b, Gates gates,
-                                                 float* __restrict__ y, int H, int G, int C) {
+                                                 Out out, int H, int G, int C) {
   constexpr int CPL = kDecodeCols, kK = 4;
   constexpr int kTileThreads = tile_threads(CPL);
   using ST = typename Storage<Tag>::T;
-  pin_args(pool, conv_pool, slot_idx, x, conv_w, conv_b, y, H, G, C);
+  pin_args(pool, conv_pool, slot_idx, x, conv_w, conv_b, H, G, C);
+  out.pin_args();
   gates.pin_args();
   const int b = blockIdx.x / G;
   const int g = blockIdx.x - b * G;
@@ -282,6 +365,8 @@ __device__ __forceinline__ void conv_decode_body(typename Storage<Tag>::T* __res
     }
 #pragma unroll
     for (int i = 0; i < kRowsPerLane; ++i) load_row(S[i], L, tile + (size_t)L.row(i) * kHD);
+    const size_t unit = (size_t)b * H + h;
+    const typename Out::Pre pre = out.load(unit, L.wave, L.lane);
     __builtin_amdgcn_sched_barrier(0);
     Gates::keep_uniform(gin);
 #pragma unroll
@@ -296,7 +381,7 @@ __device__ __forceinline__ void conv_decode_body(typename Storage<Tag>::T* __res
     }
     publish_gates(L, gates, gates.raw_of(gin), gates.consts_of(gin), lds.tile[t].gate);
     __syncthreads();
-    decode_token_from_lds<Tag, HPG>(L, S, lds, t, tile, y + ((size_t)b * H + h) * kHD);
+    decode_token_from_lds<Tag, HPG>(L, S, lds, t, tile, out, pre, unit);
   } else {
     const int slot = slot_idx[b];
     ST* tile = pool + ((size_t)slot * H + h) * (kSS * kHD);
@@ -314,7 +399,9 @@ __device__ __forceinline__ void conv_decode_body(typename Storage<Tag>::T* __res
     __syncthreads();
     publish_gates(L, gates, gates.load(b, h, 0, H, 1), GateConst{gates.A[h], gates.dt_bias[h]},
                   lds.tile[t].gate);
-    decode_token_from_lds<Tag, HPG>(L, S, lds, t, tile, y + ((size_t)b * H + h) * kHD);
+    const size_t unit = (size_t)b * H + h;
+    const typename Out::Pre pre = out.load(unit, L.wave, L.lane);
+    decode_token_from_lds<Tag, HPG>(L, S, lds, t, tile, out, pre, unit);
   }
 }
 
@@ -330,8 +417,8 @@ gdn_conv_decode_kernel(typename Storage<Tag>::T* __restrict__ pool,
                        const XT* __restrict__ x, const float* __restrict__ conv_w,
                        const float* __restrict__ conv_b, Gates gates, float* __restrict__ y,
                        int H, int G, int C) {
-  conv_decode_body<Tag, XT, Gates, HPG>(pool, conv_pool, slot_idx, x, conv_w, conv_b, gates, y,
-                                        H, G, C);
+  conv_decode_body<Tag, XT, Gates, HPG>(pool, conv_pool, slot_idx, x, conv_w, conv_b, gates,
+                                        PlainOut{y}, H, G, C);
 }
 
 template <class XT, class Gates, int HPG>
@@ -340,8 +427,23 @@ gdn_conv_decode_kernel_f32(float* __restrict__ pool, float* __restrict__ conv_po
                            const int* __restrict__ slot_idx, const XT* __restrict__ x,
                            const float* __restrict__ conv_w, const float* __restrict__ conv_b,
                            Gates gates, float* __restrict__ y, int H, int G, int C) {
-  conv_decode_body<F32, XT, Gates, HPG>(pool, conv_pool, slot_idx, x, conv_w, conv_b, gates, y,
-                                        H, G, C);
+  conv_decode_body<F32, XT, Gates, HPG>(pool, conv_pool, slot_idx, x, conv_w, conv_b, gates,
+                                        PlainOut{y}, H, G, C);
+}
+
+// The same with the gated readout (one activation type for x, the gates' raw
+// values and z).
+template <class Tag, class ATag, class Gates, int HPG>
+__global__ void __launch_bounds__(tile_threads(kDecodeCols) * HPG)
+__attribute__((amdgpu_waves_per_eu(std::is_same<Tag, F32>::value ? 1 : 4)))
+gdn_conv_decode_readout_kernel(typename Storage<Tag>::T* __restrict__ pool,
+                               float* __restrict__ conv_pool, const int* __restrict__ slot_idx,
+                               const typename ATag::T* __restrict__ x,
+                               const float* __restrict__ conv_w,
+                               const float* __restrict__ conv_b, Gates gates, GatedOut<ATag> out,
+                               int H, int G, int C) {
+  conv_decode_body<Tag, typename ATag::T, Gates, HPG>(pool, conv_pool, slot_idx, x, conv_w, conv_b,
+                                                      gates, out, H, G, C);
 }
 
 // The fp32 pool's prefill.
@@ -1970,6 +2072,94 @@ extern "C" int braid_gdn_conv_decode_raw(void* pool, int pool_dtype, int64_t n_s
                             A, dt_bias, nullptr});
   return go(RawGates<BF16>{static_cast<const uint16_t*>(a_raw),
                            static_cast<const uint16_t*>(b_raw), A, dt_bias, nullptr});
+}
+
+namespace braid {
+namespace {
+
+// One activation type for x, the raw gates and z.
+template <class ATag, class Gates>
+void launch_conv_decode_readout(void* pool, int pool_dtype, int hpg, float* conv_pool,
+                                const int32_t* slot_idx, int B, int H, int G, int C, const void* x,
+                                const float* w, const float* bias, Gates gates,
+                                GatedOut<ATag> out, hipStream_t stream) {
+  auto go = [&](auto tag, auto n) {
+    using Tag = decltype(tag);
+    constexpr int HPG = decltype(n)::value;
+    gdn_conv_decode_readout_kernel<Tag, ATag, Gates, HPG>
+        <<<dim3((unsigned)B * (unsigned)G), dim3(tile_threads(kDecodeCols) * HPG), 0, stream>>>(
+            static_cast<typename Storage<Tag>::T*>(pool), conv_pool, slot_idx,
+            static_cast<const typename ATag::T*>(x), w, bias, gates, out, H, G, C);
+  };
+  auto by_hpg = [&](auto tag) {
+    if (hpg == 1) go(tag, std::integral_constant<int, 1>{});
+    else go(tag, std::integral_constant<int, 2>{});
+  };
+  if (pool_dtype == BRAID_F32) by_hpg(F32{});
+  else if (pool_dtype == BRAID_F16) by_hpg(F16{});
+  else by_hpg(BF16{});
+}
+
+template <class ATag, class Gates>
+int conv_decode_readout(void* pool, int pool_dtype, int hpg, float* conv_pool,
+                        const int32_t* slot_idx, int B, int H, int G, int C, const void* x,
+                        const float* w, const float* bias, Gates gates, const void* z,
+                        const float* gamma, float eps, void* core, uint8_t* q, float* scale,
+                        float* partial, hipStream_t stream) {
+  using AT = typename ATag::T;
+  const GatedOut<ATag> out{static_cast<const AT*>(z), gamma, eps, static_cast<AT*>(core), partial};
+  launch_conv_decode_readout<ATag>(pool, pool_dtype, hpg, conv_pool, slot_idx, B, H, G, C, x, w,
+                                   bias, gates, out, stream);
+  if (q != nullptr) {
+    const int64_t n = (int64_t)B * H * kHD;
+    const int vec = ((reinterpret_cast<uintptr_t>(q) & 7u) == 0) ? 1 : 0;
+    quant::quantize<ATag><<<quant::blocks_for(n), quant::kThreads, 0, stream>>>(
+        out.core, partial, B * H, scale, q, n, vec);
+  }
+  const int st = hip_status(hipGetLastError(), "launching gdn_conv_decode_readout_kernel");
+  return st != BRAID_OK ? st : ok();
+}
+
+}  // namespace
+}  // namespace braid
+
+extern "C" int braid_gdn_conv_decode_readout(
+    void* pool, int pool_dtype, int64_t n_slots, int H, int G, int SS, int HD, float* conv_pool,
+    int K, const int32_t* slot_idx, int B, const void* x, const float* conv_weight,
+    const float* conv_bias, const void* a_raw, const void* b_raw, int act_dtype, const float* A,
+    const float* dt_bias, const void* z, const float* gamma, float eps, void* core, uint8_t* q,
+    float* scale, float* partial, void* stream_) {
+  hipStream_t stream = static_cast<hipStream_t>(stream_);
+  BRAID_TRY(check_common(pool, pool_dtype, n_slots, H, G, SS, HD, slot_idx, B));
+  BRAID_TRY(check_act(a_raw, b_raw, act_dtype, A, dt_bias));
+  const int hpg = H / G;
+  if (hpg != 1 && hpg != 2)
+    return fail(BRAID_EINVAL, "the fused conv decode takes 1 or 2 value heads per key group");
+  if (K != 4) return fail(BRAID_EINVAL, "the fused conv decode takes conv_kernel == 4");
+  if ((q == nullptr) != (scale == nullptr))
+    return fail(BRAID_EINVAL, "q and scale must be given together");
+  if (B == 0) return q != nullptr ? fail(BRAID_EINVAL, "x must not be empty") : ok();
+  if (conv_pool == nullptr || x == nullptr || conv_weight == nullptr)
+    return fail(BRAID_EINVAL, "conv_pool, x and conv_weight must be non-null");
+  if (!aligned16(conv_pool) || !aligned16(conv_weight))
+    return fail(BRAID_EINVAL, "conv_pool and conv_weight must be 16-byte aligned");
+  BRAID_TRY(check_dense(z, "z"));
+  BRAID_TRY(check_dense(gamma, "gamma"));
+  BRAID_TRY(check_dense(core, "core"));
+  if (partial == nullptr) return fail(BRAID_EINVAL, "partial must be non-null");
+  BRAID_TRY(validate_slots(slot_idx, B, n_slots, true, stream));
+  const int C = 2 * G * SS + H * HD;
+  if (act_dtype == BRAID_F32)
+    return conv_decode_readout<quant::XF32>(
+        pool, pool_dtype, hpg, conv_pool, slot_idx, B, H, G, C, x, conv_weight, conv_bias,
+        RawGates<F32>{static_cast<const float*>(a_raw), static_cast<const float*>(b_raw), A,
+                      dt_bias, nullptr},
+        z, gamma, eps, core, q, scale, partial, stream);
+  return conv_decode_readout<quant::XBF16>(
+      pool, pool_dtype, hpg, conv_pool, slot_idx, B, H, G, C, x, conv_weight, conv_bias,
+      RawGates<BF16>{static_cast<const uint16_t*>(a_raw), static_cast<const uint16_t*>(b_raw), A,
+                     dt_bias, nullptr},
+      z, gamma, eps, core, q, scale, partial, stream);
 }
 
 extern "C" int braid_prefill_plan_pool(const int32_t* seq_lens_host, int B, int T, int H, int cus,

@@ -267,8 +267,19 @@ quantize(const typename Tag::T* __restrict__ x, const float* __restrict__ partia
     load_vec(Tag{}, x, j * kVec, o[0]);
   }
 
+  // Four partials to a load (the workspace is 16-byte aligned wherever there
+  // are that many; checked all the same).
   float m = 0.f;
-  for (int i = threadIdx.x; i < nparts; i += kThreads) m = nan_max(m, partial[i]);
+  int i0 = 0;
+  if ((reinterpret_cast<uintptr_t>(partial) & 15u) == 0) {
+    i0 = nparts & ~3;
+    for (int i = 4 * threadIdx.x; i < i0; i += 4 * kThreads) {
+      const f32x4 p = *reinterpret_cast<const f32x4*>(partial + i);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) m = nan_max(m, p[e]);
+    }
+  }
+  for (int i = i0 + threadIdx.x; i < nparts; i += kThreads) m = nan_max(m, partial[i]);
   m = block_nan_max(m);
   const float raw = m * kInvFp8Max;
   const float sc = (raw < kEps) ? kEps : raw;

@@ -71,6 +71,9 @@ SIGNATURES = {
     "braid_gdn_conv_decode_raw": ([_vp, _i32, _i64, _i32, _i32, _i32, _i32, _vp, _i32, _vp,
                                    _i32, _vp, _i32, _vp, _vp, _vp, _vp, _i32, _vp, _vp, _vp,
                                    _vp], _i32),
+    "braid_gdn_conv_decode_readout": ([_vp, _i32, _i64, _i32, _i32, _i32, _i32, _vp, _i32, _vp,
+                                       _i32, _vp, _vp, _vp, _vp, _vp, _i32, _vp, _vp, _vp, _vp,
+                                       ctypes.c_float, _vp, _vp, _vp, _vp, _vp], _i32),
     "braid_conv1d_decode": ([_vp, _i64, _i32, _i32, _vp, _i32, _vp, _i32, _vp, _vp,
                              _vp, _vp], _i32),
     "braid_conv1d_prefill": ([_vp, _i64, _i32, _i32, _vp, _i32, _i32, _vp, _i32, _vp, _vp,
@@ -281,6 +284,55 @@ class GDNKernels:
                    HD, _ptr(conv_pool), K, _ptr(slot_idx), B, _ptr(x), _ACT_DTYPES[x.dtype],
                    _ptr(weight), bias_p, _ptr(a_raw), _ptr(b_raw), adt, _ptr(A), _ptr(dt_bias),
                    _ptr(y))
+
+    def gdn_conv_decode_readout(self, pool, conv_pool, slot_idx, x, weight, bias, a_raw, b_raw,
+                                A, dt_bias, z, gamma, eps: float, n_groups: int,
+                                quantize: bool = True):
+        """gdn_conv_decode_raw then gated_rmsnorm on its y, without y ever
+        leaving the chip, with the same bits: x [B, C], a_raw / b_raw [B, H]
+        and z (B * H * 128 elements) share one activation dtype. Returns what
+        ``gated_rmsnorm`` returns, shaped like z."""
+        pdt = _check_pool(pool, slot_idx)
+        _check(conv_pool.is_cuda and conv_pool.dtype == torch.float32
+               and conv_pool.is_contiguous() and conv_pool.dim() == 3,
+               "conv_pool must be contiguous cuda fp32 [S_max, C, K]")
+        adt = _check_raw(a_raw, b_raw, A, dt_bias)
+        n_slots, H, SS, HD = pool.shape
+        G = int(n_groups)
+        _check(G > 0 and H % G == 0, "n_heads must be divisible by n_groups")
+        C, K = conv_pool.size(1), conv_pool.size(2)
+        _check(C == 2 * G * SS + H * HD, "conv_pool channels must be 2*G*SS + H*HD")
+        _check(conv_pool.size(0) == n_slots, "conv_pool and pool must hold the same slots")
+        _check(x.dim() == 2 and x.size(1) == C, "x must be [B, C]")
+        B = x.size(0)
+        _check(x.dtype == a_raw.dtype and z.dtype == a_raw.dtype,
+               "x, a_raw, b_raw and z must share a dtype")
+        _check(x.is_cuda and x.is_contiguous(), "x must be contiguous")
+        _check(tuple(weight.shape) == (C, K), "weight must be [C, K]")
+        _check_dense_f32((weight, gamma), "weight and gamma must be contiguous cuda fp32")
+        bias_p = None
+        if bias is not None and bias.numel() > 0:
+            _check_dense_f32((bias,), "bias must be contiguous cuda fp32")
+            _check(bias.numel() == C, "bias must be [C]")
+            bias_p = _ptr(bias)
+        _check(slot_idx.numel() == B, "slot_idx must have one entry per batch row")
+        _check(a_raw.numel() == B * H and b_raw.shape == a_raw.shape, "a_raw/b_raw must be [B, H]")
+        _check(A.numel() == H and dt_bias.numel() == H, "A and dt_bias must be [H]")
+        _check(gamma.dim() == 1 and gamma.numel() == HD, "only head_dim=128 is supported")
+        _check(z.is_cuda and z.is_contiguous() and z.numel() == B * H * HD,
+               "z must be contiguous and hold B * H * HD elements")
+        core = torch.empty(z.shape, dtype=z.dtype, device=z.device)
+        partial = torch.empty(B * H, dtype=torch.float32, device=z.device)
+        q = scale = None
+        if quantize:
+            _check(B > 0, "x must not be empty")
+            q = torch.empty(z.shape, dtype=torch.float8_e4m3fn, device=z.device)
+            scale = torch.empty((1, 1), dtype=torch.float32, device=z.device)
+        self._call("braid_gdn_conv_decode_readout", pool.device, _ptr(pool), pdt, n_slots, H, G,
+                   SS, HD, _ptr(conv_pool), K, _ptr(slot_idx), B, _ptr(x), _ptr(weight), bias_p,
+                   _ptr(a_raw), _ptr(b_raw), adt, _ptr(A), _ptr(dt_bias), _ptr(z), _ptr(gamma),
+                   float(eps), _ptr(core), _ptr(q), _ptr(scale), _ptr(partial))
+        return (core, q, scale) if quantize else core
 
     @staticmethod
     def _check_decode_shapes(pool, slot_idx, q, k, v, y, B, G, SS, H, HD) -> None:

@@ -14,9 +14,10 @@ build has and the reference had not:
 * prefill's causal conv runs ``conv1d_prefill`` (one launch, window saved in
   place) instead of ``F.conv1d`` over ``[window | x]`` plus a gather
   (gdn.py:193-222); outputs and windows equal ``conv1d_decode`` token by token;
-* decode runs the conv and the recurrence as one launch
-  (``gdn_conv_decode_raw``) where the shape allows, instead of
-  ``conv1d_decode`` then ``gdn_decode_raw`` (gdn.py:131-160), same bits;
+* decode runs the conv, the recurrence and the gated norm as one launch
+  (``gdn_conv_decode_readout``) where the shape allows, instead of
+  ``conv1d_decode`` then ``gdn_decode_raw`` (gdn.py:131-160) and the torch
+  norm, same bits as the separate kernels;
 * the readout runs ``gated_rmsnorm`` (norm, gate and, for an FP8 out_proj,
   the activation quantization in two launches) instead of the torch norm and
   ``quantize_act``.
@@ -77,25 +78,34 @@ class GDNMixerLayer:
                b_raw: torch.Tensor, cache: RecurrentCache, slots_i32: torch.Tensor):
         """One token for every row: qkv_proj [B, 1, C], z [B, 1, H*HD],
         a_raw / b_raw [B, 1, H] (gdn.py:107-167 with raw gates, then _readout).
-        The conv and the recurrence run as one fused launch when the shape
-        allows it (conv kernel 4, one or two value heads per key group), with
-        the same bits as the two kernels back to back."""
+        The conv, the recurrence and the gated norm run as one fused launch when
+        the shape allows it (conv kernel 4, one or two value heads per key
+        group, one activation dtype), with the same bits as the kernels back
+        to back."""
         g = self.g
         B = qkv_proj.shape[0]
         qkv = qkv_proj[:, 0]
+        a, b = a_raw[:, 0].contiguous(), b_raw[:, 0].contiguous()
+        # One activation dtype throughout, as the kernel takes (the engine's
+        # case): the readout runs in the same launch.
+        if (self.fused_decode and qkv.dtype in (torch.float32, torch.bfloat16)
+                and a.dtype == b.dtype == z.dtype == qkv.dtype):
+            return self._mod.gdn_conv_decode_readout(
+                cache.state, cache.conv, slots_i32, qkv.contiguous(), self.conv1d_f32,
+                self.conv_bias_f32, a, b, self.A, self.dt_bias, z.contiguous(), self.norm,
+                self.eps, g.n_groups, quantize=self.fp8_out)
         y = torch.empty(B, 1, g.n_heads, g.head_dim, device=qkv.device, dtype=torch.float32)
         if self.fused_decode:
             self._mod.gdn_conv_decode_raw(cache.state, cache.conv, slots_i32, qkv.contiguous(),
-                                          self.conv1d_f32, self.conv_bias_f32,
-                                          a_raw[:, 0].contiguous(), b_raw[:, 0].contiguous(),
+                                          self.conv1d_f32, self.conv_bias_f32, a, b,
                                           self.A, self.dt_bias, y[:, 0], g.n_groups)
             return self._readout(z, y)
         conv_out = torch.empty(qkv.shape, device=qkv.device, dtype=torch.float32)
         self._mod.conv1d_decode(cache.conv, slots_i32, qkv.contiguous(), self.conv1d_f32,
                                 self.conv_bias_f32, conv_out)
         q, k, v = self._split(conv_out)
-        self._mod.gdn_decode_raw(cache.state, slots_i32, q, k, v, a_raw[:, 0].contiguous(),
-                                 b_raw[:, 0].contiguous(), self.A, self.dt_bias, y[:, 0])
+        self._mod.gdn_decode_raw(cache.state, slots_i32, q, k, v, a, b, self.A, self.dt_bias,
+                                 y[:, 0])
         return self._readout(z, y)
 
     def prefill(self, qkv_proj: torch.Tensor, z: torch.Tensor, a_raw: torch.Tensor,

@@ -165,6 +165,25 @@ int braid_gdn_conv_decode_raw(void* pool, int pool_dtype, int64_t n_slots, int H
                               const float* dt_bias, float* y, void* stream);
 
 /*
+ * braid_gdn_conv_decode_raw followed by braid_gated_rmsnorm_quant on its y, in
+ * one launch (two with q) and bit for bit the same core, codes, scale, state
+ * and windows; y is not written. x, a_raw, b_raw and z share act_dtype
+ * (BRAID_F32 or BRAID_BF16), core has it too.
+ *
+ *   z, gamma, eps, core  as braid_gated_rmsnorm_quant, units = B * H
+ *   q, scale  both NULL for the readout alone, else quantize_act(core)
+ *   partial   B * H fp32 scratch
+ */
+int braid_gdn_conv_decode_readout(void* pool, int pool_dtype, int64_t n_slots, int H, int G,
+                                  int SS, int HD, float* conv_pool, int K,
+                                  const int32_t* slot_idx, int B, const void* x,
+                                  const float* conv_weight, const float* conv_bias,
+                                  const void* a_raw, const void* b_raw, int act_dtype,
+                                  const float* A, const float* dt_bias, const void* z,
+                                  const float* gamma, float eps, void* core, uint8_t* q,
+                                  float* scale, float* partial, void* stream);
+
+/*
  * Chunk prefill scan: T tokens per launch, state held on chip between them.
  * Replaces gdn_prefill (gdn_decode.cu:553-603).
  *
