@@ -25,6 +25,7 @@
 // 128-bit accesses and a wave moves 1 KiB per instruction.
 #include "capi_common.h"
 #include "conv_common.h"
+#include "conv_prefill.h"
 
 namespace braid {
 namespace {
@@ -96,7 +97,7 @@ __global__ void __launch_bounds__(256)
 conv1d_prefill_kernel(float* __restrict__ conv_pool, const int* __restrict__ slot_idx,
                       const XT* __restrict__ x, const float* __restrict__ weight,
                       const float* __restrict__ bias, float* __restrict__ out, int C, int T,
-                      const int* __restrict__ seq_lens) {
+                      const int* __restrict__ seq_lens, bool pads) {
   constexpr int kChunk = 16;
   const int c0 = (blockIdx.x * blockDim.x + threadIdx.x) * NC;
   if (c0 >= C) return;
@@ -104,6 +105,7 @@ conv1d_prefill_kernel(float* __restrict__ conv_pool, const int* __restrict__ slo
   const int t0 = blockIdx.y * kChunk;
   int len = T;
   if (seq_lens != nullptr) len = min(max(seq_lens[b], 0), T);
+  if (!pads && t0 >= len && t0 != 0) return;
   const XT* xb = x + (size_t)b * T * C + c0;
   float* ob = out + (size_t)b * T * C + c0;
   float* st = conv_pool + ((size_t)slot_idx[b] * C + c0) * K;
@@ -150,7 +152,7 @@ conv1d_prefill_kernel(float* __restrict__ conv_pool, const int* __restrict__ slo
 #pragma unroll
       for (int j = 0; j < NC; ++j) o[j] = conv_step<K>(w[j], xs[u][j], wt[j], bias, c0 + j);
       store_out<NC>(ob + (size_t)t * C, o);
-    } else if (t < t1) {
+    } else if (pads && t < t1) {
 #pragma unroll
       for (int j = 0; j < NC; ++j) o[j] = 0.f;
       store_out<NC>(ob + (size_t)t * C, o);
@@ -202,7 +204,7 @@ int launch(int K, float* conv_pool, const int32_t* slot_idx, int B, const XT* x,
 template <class XT>
 int launch_prefill(int K, float* conv_pool, const int32_t* slot_idx, int B, int T, const XT* x,
                    const float* weight, const float* bias, float* out, int C,
-                   const int32_t* seq_lens, hipStream_t stream) {
+                   const int32_t* seq_lens, bool pads, hipStream_t stream) {
   if (T == 0) return ok();  // no tokens: nothing to compute, the windows stay as they are
   const int threads = 256;
   constexpr int kChunk = 16;
@@ -217,7 +219,7 @@ int launch_prefill(int K, float* conv_pool, const int32_t* slot_idx, int B, int 
 #define BRAID_CONV_PREFILL(KK, NC)                                                         \
   conv1d_prefill_kernel<KK, NC, XT><<<grid, threads, 0, stream>>>(conv_pool, slot_idx, x,  \
                                                                   weight, bias, out, C, T, \
-                                                                  seq_lens)
+                                                                  seq_lens, pads)
 #define BRAID_CONV_PREFILL_K(NC)              \
   switch (K) {                                \
     case 2: BRAID_CONV_PREFILL(2, NC); break; \
@@ -255,6 +257,19 @@ int check_conv(float* conv_pool, int64_t n_slots, int C, int K, const int32_t* s
 }
 
 }  // namespace
+
+int conv_prefill(float* conv_pool, int64_t n_slots, int C, int K, const int32_t* slot_idx, int B,
+                 int T, const void* x, int x_dtype, const float* weight, const float* bias,
+                 float* out, const int32_t* seq_lens, bool pads, hipStream_t stream) {
+  const int st = check_conv(conv_pool, n_slots, C, K, slot_idx, B, x, x_dtype, weight, out);
+  if (st != BRAID_OK) return st;
+  if (x_dtype == BRAID_F32)
+    return launch_prefill(K, conv_pool, slot_idx, B, T, static_cast<const float*>(x), weight,
+                          bias, out, C, seq_lens, pads, stream);
+  return launch_prefill(K, conv_pool, slot_idx, B, T, static_cast<const uint16_t*>(x), weight,
+                        bias, out, C, seq_lens, pads, stream);
+}
+
 }  // namespace braid
 
 using namespace braid;
@@ -272,11 +287,8 @@ extern "C" int braid_conv1d_prefill(float* conv_pool, int64_t n_slots, int C, in
   // would race, so (unlike the one-step decode) slots must be distinct.
   const int st = validate_slots(slot_idx, B, n_slots, true, stream);
   if (st != BRAID_OK) return st;
-  if (x_dtype == BRAID_F32)
-    return launch_prefill(K, conv_pool, slot_idx, B, T, static_cast<const float*>(x), weight,
-                          bias, out, C, seq_lens, stream);
-  return launch_prefill(K, conv_pool, slot_idx, B, T, static_cast<const uint16_t*>(x), weight,
-                        bias, out, C, seq_lens, stream);
+  return conv_prefill(conv_pool, n_slots, C, K, slot_idx, B, T, x, x_dtype, weight, bias, out,
+                      seq_lens, true, stream);
 }
 
 extern "C" int braid_conv1d_decode(float* conv_pool, int64_t n_slots, int C, int K,

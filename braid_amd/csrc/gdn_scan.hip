@@ -24,6 +24,7 @@
 
 #include "capi_common.h"
 #include "conv_common.h"
+#include "conv_prefill.h"
 #include "gated_unit.h"
 #include "gdn_mfma.h"
 #include "gdn_scan16.h"
@@ -512,7 +513,7 @@ __device__ __forceinline__ void load_stage(StageRegs<kTileWaves>& r, int wave, i
                                            const Gates& gates, const float* __restrict__ q,
                                            const float* __restrict__ k,
                                            const float* __restrict__ v, int b, int h, int g,
-                                           int H, int G, int T, int t0, int n) {
+                                           int H, int T, long qk_tok, long v_tok, int t0, int n) {
   constexpr int kThreads = 64 * kTileWaves;
   // Lane j of each of the last two waves: token j's raw gates (alpha is
   // evaluated by the first of them, beta by the second).
@@ -521,7 +522,7 @@ __device__ __forceinline__ void load_stage(StageRegs<kTileWaves>& r, int wave, i
   for (int m = 0; m < StageRegs<kTileWaves>::kV4; ++m) {
     const int e = threadIdx.x + m * kThreads, j = e / (kHD / 4), c4 = e % (kHD / 4);
     if (j < n)
-      r.v[m] = *reinterpret_cast<const float4*>(v + (((size_t)b * T + t0 + j) * H + h) * kHD +
+      r.v[m] = *reinterpret_cast<const float4*>(v + ((size_t)b * T + t0 + j) * v_tok + (size_t)h * kHD +
                                                 4 * c4);
   }
   const float* const src = ((lane >> 4) & 1) ? k : q;
@@ -530,7 +531,7 @@ __device__ __forceinline__ void load_stage(StageRegs<kTileWaves>& r, int wave, i
   for (int u = 0; u < StageRegs<kTileWaves>::kRounds; ++u) {
     const int j = wave + (2 * u + x) * kTileWaves;
     if (j < n) {
-      const float* p = src + (((size_t)b * T + t0 + j) * G + g) * kSS + e0;
+      const float* p = src + ((size_t)b * T + t0 + j) * qk_tok + (size_t)g * kSS + e0;
       r.qk[u][0] = *reinterpret_cast<const float4*>(p);
       r.qk[u][1] = *reinterpret_cast<const float4*>(p + 4);
     }
@@ -816,9 +817,9 @@ __device__ __forceinline__ void prefill_tile(float* __restrict__ pool,
                                              const float* __restrict__ q,
                                              const float* __restrict__ k,
                                              const float* __restrict__ v, const Gates& gates,
-                                             float* __restrict__ y, int H, int G,
-                                             int heads_per_group, int T, int b, int h, int part,
-                                             int len, StageLds& st) {
+                                             float* __restrict__ y, int H,
+                                             int heads_per_group, int T, long qk_tok, long v_tok,
+                                             int b, int h, int part, int len, StageLds& st) {
   using LM = typename ScanLayoutOf<Layout>::type;
   constexpr int CPL = LM::kCPL;
   constexpr int kLRG = LM::kLaneRowGroups;
@@ -842,7 +843,8 @@ __device__ __forceinline__ void prefill_tile(float* __restrict__ pool,
   const GateConst gc = gates.tile_consts(h);
   StageRegs<kW> pre;
   // (Loads nothing when len == 0; a branch around it costs ~30 VGPRs.)
-  load_stage<kW>(pre, L.wave, L.lane, gates, q, k, v, b, h, g, H, G, T, 0, min(kStage, len));
+  load_stage<kW>(pre, L.wave, L.lane, gates, q, k, v, b, h, g, H, T, qk_tok, v_tok, 0,
+                 min(kStage, len));
   for (int t0 = 0; t0 < len; t0 += kStage) {
     const int n = min(kStage, len - t0);
     // Every wave has finished reading the previous stage (the barrier at the
@@ -852,7 +854,7 @@ __device__ __forceinline__ void prefill_tile(float* __restrict__ pool,
     __syncthreads();
     // The next stage's loads fly while this stage's tokens run.
     if (t0 + kStage < len)
-      load_stage<kW>(pre, L.wave, L.lane, gates, q, k, v, b, h, g, H, G, T, t0 + kStage,
+      load_stage<kW>(pre, L.wave, L.lane, gates, q, k, v, b, h, g, H, T, qk_tok, v_tok, t0 + kStage,
                      min(kStage, len - t0 - kStage));
     float* yt = y + (((size_t)b * T + t0) * H + h) * kHD + L.col0;
     const size_t y_tok = (size_t)H * kHD;
@@ -987,7 +989,7 @@ __global__ void __launch_bounds__(64 * ScanLayoutOf<Layout>::type::kWaves)
 gdn_prefill_kernel(float* __restrict__ pool, const int* __restrict__ slot_idx,
                    const float* __restrict__ q, const float* __restrict__ k,
                    const float* __restrict__ v, Gates gates, float* __restrict__ y,
-                   int H, int G, int heads_per_group, int T) {
+                   int H, int heads_per_group, int T, long qk_tok, long v_tok) {
   using LM = typename ScanLayoutOf<Layout>::type;
   raise_scan_priority();
   const int tile_id = blockIdx.x / LM::kParts;
@@ -995,17 +997,17 @@ gdn_prefill_kernel(float* __restrict__ pool, const int* __restrict__ slot_idx,
   const int b = tile_id / H;
   const int h = tile_id - b * H;
   __shared__ StageLds st;
-  prefill_tile<Gates, Layout, Layout != 2>(pool, slot_idx, q, k, v, gates, y, H, G,
-                                                heads_per_group, T, b, h, part,
+  prefill_tile<Gates, Layout, Layout != 2>(pool, slot_idx, q, k, v, gates, y, H,
+                                                heads_per_group, T, qk_tok, v_tok, b, h, part,
                                                 gates.row_len(b, T), st);
 }
 
-template <class Tag, class Gates, int Layout>
+template <class Tag, class Gates, class YT, int Layout>
 __global__ void __launch_bounds__(Scan16Map<Layout>::kThreads)
 gdn_prefill16_kernel(uint16_t* __restrict__ pool, const int* __restrict__ slot_idx,
                      const float* __restrict__ q, const float* __restrict__ k,
-                     const float* __restrict__ v, Gates gates, float* __restrict__ y, int H, int G,
-                     int heads_per_group, int T) {
+                     const float* __restrict__ v, Gates gates, YT* __restrict__ y, int H,
+                     int heads_per_group, int T, long qk_tok, long v_tok) {
   constexpr int kParts = Scan16Map<Layout>::kParts;
   raise_scan_priority();
   const int tile_id = blockIdx.x / kParts;
@@ -1013,8 +1015,8 @@ gdn_prefill16_kernel(uint16_t* __restrict__ pool, const int* __restrict__ slot_i
   const int b = tile_id / H;
   const int h = tile_id - b * H;
   __shared__ Scan16Lds<Tag, Layout> lds;
-  prefill_tile16<Tag, Gates, Layout>(pool, slot_idx, q, k, v, gates, y, H, G, heads_per_group, T,
-                                     b, h, part, gates.row_len(b, T), lds);
+  prefill_tile16<Tag, Gates, YT, Layout>(pool, slot_idx, q, k, v, gates, y, H, heads_per_group, T,
+                                         qk_tok, v_tok, b, h, part, gates.row_len(b, T), lds);
 }
 
 // A token's time in each tier of the planned kernel, us (MI355X, one workgroup
@@ -1042,12 +1044,12 @@ constexpr int kPlans = (kMaxN8 + 1) * (kMaxN4 + 1) * (kMaxN2 + 1);
 // of its longest row's time and its total time over the CUs, within max_extra
 // workgroups beyond one per tile (what the grid has room for). The grid's
 // workgroups beyond the plan return. A row's bits do not depend on its tier.
-template <class Tag, class Gates>
+template <class Tag, class Gates, class YT>
 __global__ void __launch_bounds__(Scan16Map<2>::kThreads)
 gdn_prefill16_planned_kernel(uint16_t* __restrict__ pool, const int* __restrict__ slot_idx,
                              const float* __restrict__ q, const float* __restrict__ k,
-                             const float* __restrict__ v, Gates gates, float* __restrict__ y,
-                             int B, int H, int G, int heads_per_group, int T, int cus,
+                             const float* __restrict__ v, Gates gates, YT* __restrict__ y, int B,
+                             int H, int heads_per_group, int T, long qk_tok, long v_tok, int cus,
                              int max_extra, int plan) {
   raise_scan_priority();
   union Lds {
@@ -1131,17 +1133,17 @@ gdn_prefill16_planned_kernel(uint16_t* __restrict__ pool, const int* __restrict_
   if (b < 0) return;
   Lds& lds = *reinterpret_cast<Lds*>(smem);
   if (tier == 0)
-    prefill_tile16<Tag, Gates, 8, true>(pool, slot_idx, q, k, v, gates, y, H, G, heads_per_group,
-                                        T, b, i >> 3, i & 7, len, lds.l8);
+    prefill_tile16<Tag, Gates, YT, 8, true>(pool, slot_idx, q, k, v, gates, y, H,
+                                            heads_per_group, T, qk_tok, v_tok, b, i >> 3, i & 7, len, lds.l8);
   else if (tier == 1)
-    prefill_tile16<Tag, Gates, 4, true>(pool, slot_idx, q, k, v, gates, y, H, G, heads_per_group,
-                                        T, b, i >> 2, i & 3, len, lds.l4);
+    prefill_tile16<Tag, Gates, YT, 4, true>(pool, slot_idx, q, k, v, gates, y, H,
+                                            heads_per_group, T, qk_tok, v_tok, b, i >> 2, i & 3, len, lds.l4);
   else if (tier == 2)
-    prefill_tile16<Tag, Gates, 1, true>(pool, slot_idx, q, k, v, gates, y, H, G, heads_per_group,
-                                        T, b, i >> 1, i & 1, len, lds.l1);
+    prefill_tile16<Tag, Gates, YT, 1, true>(pool, slot_idx, q, k, v, gates, y, H,
+                                            heads_per_group, T, qk_tok, v_tok, b, i >> 1, i & 1, len, lds.l1);
   else
-    prefill_tile16<Tag, Gates, 2, true>(pool, slot_idx, q, k, v, gates, y, H, G, heads_per_group,
-                                        T, b, i, 0, len, lds.l2);
+    prefill_tile16<Tag, Gates, YT, 2, true>(pool, slot_idx, q, k, v, gates, y, H,
+                                            heads_per_group, T, qk_tok, v_tok, b, i, 0, len, lds.l2);
 }
 
 // Ragged batches on an fp32 pool, of up to four tiles per CU: the rows' live lengths decide
@@ -1168,8 +1170,8 @@ __global__ void __launch_bounds__(256)
 gdn_prefill_planned_kernel(float* __restrict__ pool, const int* __restrict__ slot_idx,
                            const float* __restrict__ q, const float* __restrict__ k,
                            const float* __restrict__ v, Gates gates, float* __restrict__ y,
-                           int B, int H, int G, int heads_per_group, int T, int cus,
-                           int max_extra, int forced_plan) {
+                           int B, int H, int heads_per_group, int T, long qk_tok, long v_tok,
+                           int cus, int max_extra, int forced_plan) {
   raise_scan_priority();
   __shared__ StageLds st;
   __shared__ int lens[kMaxPlanRows];
@@ -1238,23 +1240,24 @@ gdn_prefill_planned_kernel(float* __restrict__ pool, const int* __restrict__ slo
   if (i < 8 * n8 * H) {
     const int rank = i / (8 * H), rem = i - rank * 8 * H;
     const int b = order[rank];
-    prefill_tile<Gates, 8, true>(pool, slot_idx, q, k, v, gates, y, H, G, heads_per_group, T,
-                                      b, rem >> 3, rem & 7, lens[b], st);
+    prefill_tile<Gates, 8, true>(pool, slot_idx, q, k, v, gates, y, H, heads_per_group, T,
+                                qk_tok, v_tok, b, rem >> 3, rem & 7, lens[b], st);
     return;
   }
   i -= 8 * n8 * H;
   if (i < 4 * n4 * H) {
     const int rank = n8 + i / (4 * H), rem = i - (rank - n8) * 4 * H;
     const int b = order[rank];
-    prefill_tile<Gates, 4, true>(pool, slot_idx, q, k, v, gates, y, H, G, heads_per_group, T,
-                                      b, rem >> 2, rem & 3, lens[b], st);
+    prefill_tile<Gates, 4, true>(pool, slot_idx, q, k, v, gates, y, H, heads_per_group, T,
+                                qk_tok, v_tok, b, rem >> 2, rem & 3, lens[b], st);
     return;
   }
   i -= 4 * n4 * H;
   if (i < 2 * n2 * H) {
     const int rank = n8 + n4 + i / (2 * H), rem = i - (rank - n8 - n4) * 2 * H;
     const int b = order[rank];
-    prefill_tile<Gates, 1>(pool, slot_idx, q, k, v, gates, y, H, G, heads_per_group, T, b,
+    prefill_tile<Gates, 1>(pool, slot_idx, q, k, v, gates, y, H, heads_per_group, T,
+                                qk_tok, v_tok, b,
                                 rem >> 1, rem & 1, lens[b], st);
     return;
   }
@@ -1262,7 +1265,8 @@ gdn_prefill_planned_kernel(float* __restrict__ pool, const int* __restrict__ slo
   if (i < (B - n8 - n4 - n2) * H) {
     const int rank = n8 + n4 + n2 + i / H;
     const int b = order[rank];
-    prefill_tile<Gates, 2>(pool, slot_idx, q, k, v, gates, y, H, G, heads_per_group, T, b,
+    prefill_tile<Gates, 2>(pool, slot_idx, q, k, v, gates, y, H, heads_per_group, T,
+                                qk_tok, v_tok, b,
                                 i - (i / H) * H, 0, lens[b], st);
   }
 }
@@ -1428,21 +1432,28 @@ int prefill_layout(int n_tiles, int B, int T, bool ragged, int cus) {
   return ragged && B <= kMaxPlanRows && cus > 0 && n_tiles <= 4 * cus ? 0 : 2;
 }
 
+// A prefill's q, k and v: token t of row b of q (k, v) starts at q + (b * T + t)
+// * qk_tok (v + ... * v_tok); a token's heads are dense.
+struct ScanIn {
+  const float *q, *k, *v;
+  long qk_tok, v_tok;
+};
+
 // fp32 pools.
 template <class Gates, int Layout>
 void launch_prefill_cols(void* pool, const int32_t* slot_idx, int B, int T, int H, int G,
-                         const float* q, const float* k, const float* v, Gates gates, float* y,
-                         hipStream_t stream) {
+                         const ScanIn& in, Gates gates, float* y, hipStream_t stream) {
   using LM = typename ScanLayoutOf<Layout>::type;
   const dim3 grid((unsigned)B * (unsigned)H * LM::kParts), block(64 * LM::kWaves);
   gdn_prefill_kernel<Gates, Layout><<<grid, block, 0, stream>>>(
-      static_cast<float*>(pool), slot_idx, q, k, v, gates, y, H, G, H / G, T);
+      static_cast<float*>(pool), slot_idx, in.q, in.k, in.v, gates, y, H, H / G, T, in.qk_tok,
+      in.v_tok);
 }
 
 template <class Gates>
 void launch_prefill_planned(void* pool, const int32_t* slot_idx, int B, int T,
-                            int H, int G, const float* q, const float* k, const float* v,
-                            Gates gates, float* y, int cus, int forced, hipStream_t stream) {
+                            int H, int G, const ScanIn& in, Gates gates, float* y, int cus,
+                            int forced, hipStream_t stream) {
   // At most one extra workgroup per CU for split tiles; the grid has room for
   // whatever the plan uses (the rest return at once).
   const int max_extra = std::min(cus, 3 * B * H);
@@ -1456,8 +1467,8 @@ void launch_prefill_planned(void* pool, const int32_t* slot_idx, int B, int T,
   }
   const dim3 grid((unsigned)n_wg), block(256);
   gdn_prefill_planned_kernel<Gates><<<grid, block, 0, stream>>>(
-      static_cast<float*>(pool), slot_idx, q, k, v, gates, y, B, H, G, H / G, T, cus, max_extra,
-      forced);
+      static_cast<float*>(pool), slot_idx, in.q, in.k, in.v, gates, y, B, H, H / G, T, in.qk_tok,
+      in.v_tok, cus, max_extra, forced);
 }
 
 // Host plan of a ragged prefill (the planned kernel's tiers), from the live
@@ -1725,22 +1736,21 @@ int prefill_layout16(int n_tiles, int B, bool ragged, int cus) {
   return 2;
 }
 
-template <class Tag, class Gates>
+template <class Tag, class Gates, class YT>
 void launch_prefill16(void* pool, int pool_dtype, const int32_t* slot_idx, int B, int T, int H,
-                      int G, const float* q, const float* k, const float* v, Gates gates, float* y,
-                      const std::vector<int32_t>* host_lens, int plan_hint, hipStream_t stream) {
+                      int G, const ScanIn& in, Gates gates, YT* y, const std::vector<int32_t>* host_lens, int plan_hint, hipStream_t stream) {
   const int cus = device_cus();
   uint16_t* const p = static_cast<uint16_t*>(pool);
   const int layout = prefill_layout16(B * H, B, gates.ragged(), cus);
   auto run = [&](auto kern, int parts, int threads) {
     kern<<<dim3((unsigned)B * (unsigned)H * (unsigned)parts), dim3(threads), 0, stream>>>(
-        p, slot_idx, q, k, v, gates, y, H, G, H / G, T);
+        p, slot_idx, in.q, in.k, in.v, gates, y, H, H / G, T, in.qk_tok, in.v_tok);
   };
   auto run_layout = [&](int l) {
-    if (l == 8) run(gdn_prefill16_kernel<Tag, Gates, 8>, 8, Scan16Map<8>::kThreads);
-    else if (l == 4) run(gdn_prefill16_kernel<Tag, Gates, 4>, 4, Scan16Map<4>::kThreads);
-    else if (l == 1) run(gdn_prefill16_kernel<Tag, Gates, 1>, 2, Scan16Map<1>::kThreads);
-    else run(gdn_prefill16_kernel<Tag, Gates, 2>, 1, Scan16Map<2>::kThreads);
+    if (l == 8) run(gdn_prefill16_kernel<Tag, Gates, YT, 8>, 8, Scan16Map<8>::kThreads);
+    else if (l == 4) run(gdn_prefill16_kernel<Tag, Gates, YT, 4>, 4, Scan16Map<4>::kThreads);
+    else if (l == 1) run(gdn_prefill16_kernel<Tag, Gates, YT, 1>, 2, Scan16Map<1>::kThreads);
+    else run(gdn_prefill16_kernel<Tag, Gates, YT, 2>, 1, Scan16Map<2>::kThreads);
   };
   if (layout != 0) return run_layout(layout);
   // The PREFILL_PLAN knob (measurement), else the host's plan from lengths it
@@ -1761,26 +1771,31 @@ void launch_prefill16(void* pool, int pool_dtype, const int32_t* slot_idx, int B
       return run_layout(n8 == B ? 8 : (n4 == B ? 4 : (n2 == B ? 1 : 2)));
     n_wg = (B + 7 * n8 + 3 * n4 + n2) * H;
   }
-  gdn_prefill16_planned_kernel<Tag, Gates>
+  gdn_prefill16_planned_kernel<Tag, Gates, YT>
       <<<dim3((unsigned)n_wg), dim3(Scan16Map<2>::kThreads), 0, stream>>>(
-          p, slot_idx, q, k, v, gates, y, B, H, G, H / G, T, some_cus, max_extra, plan);
+          p, slot_idx, in.q, in.k, in.v, gates, y, B, H, H / G, T, in.qk_tok, in.v_tok, some_cus,
+          max_extra, plan);
 }
 
-template <class Gates>
+// y: fp32, or (16-bit pools, bf16 gates) bf16.
+template <class Gates, class YT>
 int launch_prefill(void* pool, int pool_dtype, const int32_t* slot_idx, int B, int T, int H,
-                   int G, const float* q, const float* k, const float* v, Gates gates,
-                   float* y, const std::vector<int32_t>* host_lens, hipStream_t stream,
+                   int G, const ScanIn& in, Gates gates, YT* y,
+                   const std::vector<int32_t>* host_lens, hipStream_t stream,
                    int plan_hint = -1) {
   if (pool_dtype != BRAID_F32) {
     if (pool_dtype == BRAID_F16)
-      launch_prefill16<F16>(pool, pool_dtype, slot_idx, B, T, H, G, q, k, v, gates, y, host_lens,
+      launch_prefill16<F16>(pool, pool_dtype, slot_idx, B, T, H, G, in, gates, y, host_lens,
                             plan_hint, stream);
     else
-      launch_prefill16<BF16>(pool, pool_dtype, slot_idx, B, T, H, G, q, k, v, gates, y, host_lens,
+      launch_prefill16<BF16>(pool, pool_dtype, slot_idx, B, T, H, G, in, gates, y, host_lens,
                              plan_hint, stream);
     const int st = hip_status(hipGetLastError(), "launching gdn_prefill16_kernel");
     return st != BRAID_OK ? st : ok();
   }
+  if constexpr (!std::is_same<YT, float>::value) {
+    return fail(BRAID_EINVAL, "an fp32 pool's scan writes fp32 y");
+  } else {
   const int cus = device_cus();
   int layout = prefill_layout(B * H, B, T, gates.ragged(), cus);
   // With the live lengths on the host, every ragged batch the planned kernel
@@ -1807,23 +1822,24 @@ int launch_prefill(void* pool, int pool_dtype, const int32_t* slot_idx, int B, i
     layout = n8 == B ? 8 : (n4 == B ? 4 : (n2 == B ? 1 : 0));
   }
   if (layout == 8)
-    launch_prefill_cols<Gates, 8>(pool, slot_idx, B, T, H, G, q, k, v, gates, y, stream);
+    launch_prefill_cols<Gates, 8>(pool, slot_idx, B, T, H, G, in, gates, y, stream);
   else if (layout == 4)
-    launch_prefill_cols<Gates, 4>(pool, slot_idx, B, T, H, G, q, k, v, gates, y, stream);
+    launch_prefill_cols<Gates, 4>(pool, slot_idx, B, T, H, G, in, gates, y, stream);
   else if (layout == 1)
-    launch_prefill_cols<Gates, 1>(pool, slot_idx, B, T, H, G, q, k, v, gates, y, stream);
+    launch_prefill_cols<Gates, 1>(pool, slot_idx, B, T, H, G, in, gates, y, stream);
   else if (layout == 2)
-    launch_prefill_cols<Gates, 2>(pool, slot_idx, B, T, H, G, q, k, v, gates, y, stream);
+    launch_prefill_cols<Gates, 2>(pool, slot_idx, B, T, H, G, in, gates, y, stream);
   else {
     // The PREFILL_PLAN knob (measurement) forces a plan; otherwise an eager
     // call runs the host's plan and a captured one leaves it to the kernel.
     int forced = launch_knob(BRAID_KNOB_PREFILL_PLAN);
     if (forced < 0) forced = host_plan;
-    launch_prefill_planned<Gates>(pool, slot_idx, B, T, H, G, q, k, v, gates, y,
+    launch_prefill_planned<Gates>(pool, slot_idx, B, T, H, G, in, gates, y,
                                   cus > 0 ? cus : 256, forced, stream);
   }
   const int st = hip_status(hipGetLastError(), "launching gdn_prefill_kernel");
   return st != BRAID_OK ? st : ok();
+  }
 }
 
 int check_dense(const void* p, const char* name) {
@@ -1908,7 +1924,8 @@ extern "C" int braid_gdn_prefill(void* pool, int pool_dtype, int64_t n_slots, in
       return fail(BRAID_EINVAL, "alpha/beta must be non-null");
   }
   BRAID_TRY(validate_slots(slot_idx, B, n_slots, true, stream));
-  return launch_prefill(pool, pool_dtype, slot_idx, B, T, H, G, q, k, v,
+  return launch_prefill(pool, pool_dtype, slot_idx, B, T, H, G,
+                        ScanIn{q, k, v, (long)G * SS, (long)H * HD},
                         PrecomputedGates{alpha, beta}, y, nullptr, stream);
 }
 
@@ -1942,16 +1959,17 @@ int prefill_raw(void* pool, int pool_dtype, int64_t n_slots, int H, int G, int S
                            host_lens.empty() ? nullptr : seq_lens,
                            host_lens.empty() ? nullptr : host_lens.data()));
   const std::vector<int32_t>* lens_p = host_lens.empty() ? nullptr : &host_lens;
+  const ScanIn in{q, k, v, (long)G * SS, (long)H * HD};
   if (act_dtype == BRAID_F32) {
     RawGates<F32> gates{static_cast<const float*>(a_raw), static_cast<const float*>(b_raw), A,
                         dt_bias, seq_lens};
-    return launch_prefill(pool, pool_dtype, slot_idx, B, T, H, G, q, k, v, gates, y, lens_p,
-                          stream, plan_hint);
+    return launch_prefill(pool, pool_dtype, slot_idx, B, T, H, G, in, gates, y, lens_p, stream,
+                          plan_hint);
   }
   RawGates<BF16> gates{static_cast<const uint16_t*>(a_raw), static_cast<const uint16_t*>(b_raw),
                        A, dt_bias, seq_lens};
-  return launch_prefill(pool, pool_dtype, slot_idx, B, T, H, G, q, k, v, gates, y, lens_p,
-                        stream, plan_hint);
+  return launch_prefill(pool, pool_dtype, slot_idx, B, T, H, G, in, gates, y, lens_p, stream,
+                        plan_hint);
 }
 
 }  // namespace
@@ -1977,6 +1995,54 @@ extern "C" int braid_gdn_prefill_raw_plan(void* pool, int pool_dtype, int64_t n_
     return fail(BRAID_EINVAL, "a prefill plan needs seq_lens (it plans ragged batches)");
   return prefill_raw(pool, pool_dtype, n_slots, H, G, SS, HD, slot_idx, B, T, q, k, v, a_raw,
                      b_raw, act_dtype, A, dt_bias, y, seq_lens, plan, stream_);
+}
+
+extern "C" int braid_gdn_conv_prefill_raw(
+    void* pool, int pool_dtype, int64_t n_slots, int H, int G, int SS, int HD, float* conv_pool,
+    int K, const int32_t* slot_idx, int B, int T, const void* x, int x_dtype,
+    const float* conv_weight, const float* conv_bias, float* conv_out, const void* a_raw,
+    const void* b_raw, int act_dtype, const float* A, const float* dt_bias, void* y, int y_dtype,
+    const int32_t* seq_lens, int plan, void* stream_) {
+  hipStream_t stream = static_cast<hipStream_t>(stream_);
+  BRAID_TRY(check_common(pool, pool_dtype, n_slots, H, G, SS, HD, slot_idx, B));
+  if (T < 0) return fail(BRAID_EINVAL, "T must be non-negative");
+  BRAID_TRY(check_act(a_raw, b_raw, act_dtype, A, dt_bias));
+  const int C = 2 * G * SS + H * HD;
+  if (plan >= 0 && seq_lens == nullptr)
+    return fail(BRAID_EINVAL, "a prefill plan needs seq_lens (it plans ragged batches)");
+  if (y_dtype != BRAID_F32 &&
+      !(y_dtype == BRAID_BF16 && act_dtype == BRAID_BF16 && pool_dtype != BRAID_F32))
+    return fail(BRAID_EINVAL, "y is fp32, or bf16 with bf16 gates on a 16-bit pool");
+  if (B == 0) return ok();
+  if (T > 0) {
+    BRAID_TRY(check_dense(conv_out, "conv_out"));
+    BRAID_TRY(check_dense(y, "y"));
+  }
+  // One slot check for both kernels, with the lengths for the scan's plan.
+  std::vector<int32_t> host_lens;
+  int cap_st = BRAID_OK;
+  const bool capturing = stream_capturing(stream, &cap_st);
+  if (cap_st != BRAID_OK) return cap_st;
+  if (seq_lens != nullptr && !capturing && T > 0) host_lens.resize(B);
+  BRAID_TRY(validate_slots(slot_idx, B, n_slots, true, stream,
+                           host_lens.empty() ? nullptr : seq_lens,
+                           host_lens.empty() ? nullptr : host_lens.data()));
+  const std::vector<int32_t>* lens_p = host_lens.empty() ? nullptr : &host_lens;
+  BRAID_TRY(conv_prefill(conv_pool, n_slots, C, K, slot_idx, B, T, x, x_dtype, conv_weight,
+                         conv_bias, conv_out, seq_lens, /*pads=*/false, stream));
+  const ScanIn in{conv_out, conv_out + (size_t)G * SS, conv_out + (size_t)2 * G * SS, C, C};
+  if (act_dtype == BRAID_F32)
+    return launch_prefill(pool, pool_dtype, slot_idx, B, T, H, G, in,
+                          RawGates<F32>{static_cast<const float*>(a_raw),
+                                        static_cast<const float*>(b_raw), A, dt_bias, seq_lens},
+                          static_cast<float*>(y), lens_p, stream, plan);
+  const RawGates<BF16> gates{static_cast<const uint16_t*>(a_raw),
+                             static_cast<const uint16_t*>(b_raw), A, dt_bias, seq_lens};
+  if (y_dtype == BRAID_BF16)
+    return launch_prefill(pool, pool_dtype, slot_idx, B, T, H, G, in, gates,
+                          static_cast<uint16_t*>(y), lens_p, stream, plan);
+  return launch_prefill(pool, pool_dtype, slot_idx, B, T, H, G, in, gates,
+                        static_cast<float*>(y), lens_p, stream, plan);
 }
 
 namespace braid {
@@ -2113,8 +2179,10 @@ int conv_decode_readout(void* pool, int pool_dtype, int hpg, float* conv_pool,
   if (q != nullptr) {
     const int64_t n = (int64_t)B * H * kHD;
     const int vec = ((reinterpret_cast<uintptr_t>(q) & 7u) == 0) ? 1 : 0;
-    quant::quantize<ATag><<<quant::blocks_for(n), quant::kThreads, 0, stream>>>(
-        out.core, partial, B * H, scale, q, n, vec);
+    auto* const kern = B * H > quant::kThreads && aligned16(partial) ? quant::quantize<ATag, true>
+                                                                     : quant::quantize<ATag>;
+    kern<<<quant::blocks_for(n), quant::kThreads, 0, stream>>>(out.core, partial, B * H, scale, q,
+                                                               n, vec);
   }
   const int st = hip_status(hipGetLastError(), "launching gdn_conv_decode_readout_kernel");
   return st != BRAID_OK ? st : ok();

@@ -379,15 +379,21 @@ __device__ __forceinline__ float token16(const Scan16Map<Layout>& L, State16<Tag
 // what the scan is short of, and a stage's preparation (norms, parts, gates) is
 // a long chain with many waits; on waves of its own it runs beside the tokens,
 // one stage ahead, and meets them at one barrier a stage.
-template <class Tag, class Gates, int Layout, bool kTight = false>
+// y's element from its fp32 value: as it is, or rounded to bf16 (the readout's
+// first step, for callers that would do it next).
+__device__ __forceinline__ void put_y(float* p, float y) { *p = y; }
+__device__ __forceinline__ void put_y(uint16_t* p, float y) { *p = (uint16_t)pack_bf16x2(y, 0.f); }
+
+template <class Tag, class Gates, class YT, int Layout, bool kTight = false>
 __device__ __forceinline__ void prefill_tile16(uint16_t* __restrict__ pool,
                                                const int* __restrict__ slot_idx,
                                                const float* __restrict__ q,
                                                const float* __restrict__ k,
                                                const float* __restrict__ v, const Gates& gates,
-                                               float* __restrict__ y, int H, int G,
-                                               int heads_per_group, int T, int b, int h, int part,
-                                               int len, Scan16Lds<Tag, Layout>& lds) {
+                                               YT* __restrict__ y, int H,
+                                               int heads_per_group, int T, long qk_tok, long v_tok,
+                                               int b, int h, int part, int len,
+                                               Scan16Lds<Tag, Layout>& lds) {
   using LM = Scan16Map<Layout>;
   using St = Stage16<Tag, Layout>;
   constexpr int kWgCols = LM::kWaves * LM::kCols;
@@ -398,8 +404,10 @@ __device__ __forceinline__ void prefill_tile16(uint16_t* __restrict__ pool,
   // A layout's waves beyond kThreads (the planned kernel launches the most any
   // layout needs) end here; the workgroup's barriers count the live ones.
   if (wave >= LM::kWaves + LM::kPrep) return;
-  const Scan16Row in{q + ((size_t)b * T * G + g) * kSS, k + ((size_t)b * T * G + g) * kSS,
-                     v + ((size_t)b * T * H + h) * kHD + c0, (size_t)G * kSS, (size_t)H * kHD};
+  const Scan16Row in{q + (size_t)b * T * qk_tok + (size_t)g * kSS,
+                     k + (size_t)b * T * qk_tok + (size_t)g * kSS,
+                     v + (size_t)b * T * v_tok + (size_t)h * kHD + c0, (size_t)qk_tok,
+                     (size_t)v_tok};
   auto gate_slot = [&](int s) {
     return &lds.gate[(s / kGateStages) & 1][(s % kGateStages) * kStage16];
   };
@@ -450,7 +458,7 @@ __device__ __forceinline__ void prefill_tile16(uint16_t* __restrict__ pool,
     asm("" : "+v"(neg_zero));
     const size_t y_tok = (size_t)H * kHD;
     // Where the lane's y goes: its slot's token of each kSlots tokens.
-    float* yp = y + (((size_t)b * T + L.slot) * H + h) * kHD + c0 + L.col;
+    YT* yp = y + (((size_t)b * T + L.slot) * H + h) * kHD + c0 + L.col;
     float yv = 0.f;
     int stage = 0;
     for (int t0 = 0; t0 < len; t0 += kStage16, ++stage) {
@@ -482,7 +490,7 @@ __device__ __forceinline__ void prefill_tile16(uint16_t* __restrict__ pool,
 #pragma unroll
         for (int i = 0; i < 4; ++i) step(j + i, i & 1);
         if (((j + 4) & (LM::kSlots - 1)) == 0) {
-          *yp = yv;
+          put_y(yp, yv);
           yp += LM::kSlots * y_tok;
         }
       }
@@ -494,18 +502,16 @@ __device__ __forceinline__ void prefill_tile16(uint16_t* __restrict__ pool,
       __syncthreads();
     }
     const int rest = len & (LM::kSlots - 1);
-    if (L.slot < rest) *yp = yv;
+    if (L.slot < rest) put_y(yp, yv);
     S.store(L, tile);
   }
 
   // Zeros at the pad positions, the workgroup's columns, 16 bytes per thread.
-  constexpr int kV4 = kWgCols / 4;
-  for (int e = threadIdx.x; e < (T - len) * kV4; e += LM::kThreads) {
-    const int t = len + e / kV4, c = c0 + 4 * (e % kV4);
-    typedef float f32x4 __attribute__((ext_vector_type(4)));
-    __builtin_nontemporal_store(
-        (f32x4){0.f, 0.f, 0.f, 0.f},
-        reinterpret_cast<f32x4*>(y + (((size_t)b * T + t) * H + h) * kHD + c));
+  constexpr int kPer = 16 / sizeof(YT), kV = kWgCols / kPer;
+  for (int e = threadIdx.x; e < (T - len) * kV; e += LM::kThreads) {
+    const int t = len + e / kV, c = c0 + kPer * (e % kV);
+    __builtin_nontemporal_store((u32x4){0u, 0u, 0u, 0u},
+                                reinterpret_cast<u32x4*>(y + (((size_t)b * T + t) * H + h) * kHD + c));
   }
 }
 

@@ -249,7 +249,9 @@ __device__ __forceinline__ void store_codes(uint8_t* p, uint2 v) {
 // reduced to the scale, so the reduction overlaps them: kUnroll vectors a
 // thread when it has that many, else its first vector (a [64, 4096] input
 // gives each thread one).
-template <class Tag>
+// kPartVec: the partials, 16-byte aligned, are read four to a load (for
+// producers that leave more than one per thread).
+template <class Tag, bool kPartVec = false>
 __global__ void __launch_bounds__(kThreads)
 quantize(const typename Tag::T* __restrict__ x, const float* __restrict__ partial, int nparts,
          float* __restrict__ scale, uint8_t* __restrict__ q, long n, int vec) {
@@ -267,11 +269,9 @@ quantize(const typename Tag::T* __restrict__ x, const float* __restrict__ partia
     load_vec(Tag{}, x, j * kVec, o[0]);
   }
 
-  // Four partials to a load (the workspace is 16-byte aligned wherever there
-  // are that many; checked all the same).
   float m = 0.f;
   int i0 = 0;
-  if ((reinterpret_cast<uintptr_t>(partial) & 15u) == 0) {
+  if constexpr (kPartVec) {
     i0 = nparts & ~3;
     for (int i = 4 * threadIdx.x; i < i0; i += 4 * kThreads) {
       const f32x4 p = *reinterpret_cast<const f32x4*>(partial + i);

@@ -74,6 +74,9 @@ SIGNATURES = {
     "braid_gdn_conv_decode_readout": ([_vp, _i32, _i64, _i32, _i32, _i32, _i32, _vp, _i32, _vp,
                                        _i32, _vp, _vp, _vp, _vp, _vp, _i32, _vp, _vp, _vp, _vp,
                                        ctypes.c_float, _vp, _vp, _vp, _vp, _vp], _i32),
+    "braid_gdn_conv_prefill_raw": ([_vp, _i32, _i64, _i32, _i32, _i32, _i32, _vp, _i32, _vp, _i32,
+                                    _i32, _vp, _i32, _vp, _vp, _vp, _vp, _vp, _i32, _vp, _vp, _vp,
+                                    _i32, _vp, _i32, _vp], _i32),
     "braid_conv1d_decode": ([_vp, _i64, _i32, _i32, _vp, _i32, _vp, _i32, _vp, _vp,
                              _vp, _vp], _i32),
     "braid_conv1d_prefill": ([_vp, _i64, _i32, _i32, _vp, _i32, _i32, _vp, _i32, _vp, _vp,
@@ -391,6 +394,59 @@ class GDNKernels:
         self._call("braid_gdn_prefill_raw_plan", pool.device, _ptr(pool), pdt, pool.size(0), H,
                    G, SS, HD, _ptr(slot_idx), B, T, _ptr(q), _ptr(k), _ptr(v), _ptr(a_raw),
                    _ptr(b_raw), adt, _ptr(A), _ptr(dt_bias), _ptr(y), _ptr(seq_lens), plan)
+
+    def gdn_conv_prefill_raw(self, pool, conv_pool, slot_idx, x, weight, bias, a_raw, b_raw, A,
+                             dt_bias, y, n_groups: int,
+                             seq_lens: Optional[torch.Tensor] = None,
+                             plan_lens: Optional[Sequence[int]] = None) -> None:
+        """conv1d_prefill then gdn_prefill_raw on its output's q/k/v columns,
+        read in place, behind one slot check; the same bits. x [B, T, C]; y
+        [B, T, H, HD] fp32, or bf16 (with bf16 gates and a 16-bit pool): the
+        same values rounded as the readout rounds them."""
+        pdt = _check_pool(pool, slot_idx)
+        _check(conv_pool.is_cuda and conv_pool.dtype == torch.float32
+               and conv_pool.is_contiguous() and conv_pool.dim() == 3,
+               "conv_pool must be contiguous cuda fp32 [S_max, C, K]")
+        adt = _check_raw(a_raw, b_raw, A, dt_bias)
+        n_slots, H, SS, HD = pool.shape
+        G = int(n_groups)
+        _check(SS == 128 and HD == 128, "only SS=HD=128 is instantiated")
+        _check(G > 0 and H % G == 0, "n_heads must be divisible by n_groups")
+        C, K = conv_pool.size(1), conv_pool.size(2)
+        _check(C == 2 * G * SS + H * HD, "conv_pool channels must be 2*G*SS + H*HD")
+        _check(conv_pool.size(0) == n_slots, "conv_pool and pool must hold the same slots")
+        _check(x.dim() == 3 and x.size(2) == C, "x must be [B, T, C]")
+        B, T = x.size(0), x.size(1)
+        _check(x.dtype in _ACT_DTYPES, "x must be fp32 or bf16 (the activation dtypes braid runs)")
+        _check(x.is_cuda and x.is_contiguous(), "x must be contiguous")
+        _check(tuple(weight.shape) == (C, K), "weight must be [C, K]")
+        _check_dense_f32((weight,), "weight must be contiguous cuda fp32")
+        bias_p = None
+        if bias is not None and bias.numel() > 0:
+            _check_dense_f32((bias,), "bias must be contiguous cuda fp32")
+            _check(bias.numel() == C, "bias must be [C]")
+            bias_p = _ptr(bias)
+        _check(slot_idx.numel() == B, "slot_idx must have one entry per batch row")
+        _check(a_raw.dim() >= 2 and a_raw.size(0) == B and a_raw.size(1) == T
+               and a_raw.numel() == B * T * H, "a_raw must be [B, T, H]")
+        _check(b_raw.shape == a_raw.shape, "b_raw must match a_raw")
+        _check(A.numel() == H and dt_bias.numel() == H, "A and dt_bias must be [H]")
+        _check(y.is_cuda and y.is_contiguous() and tuple(y.shape) == (B, T, H, HD)
+               and y.dtype in _ACT_DTYPES, "y must be contiguous cuda fp32 or bf16 [B, T, H, HD]")
+        plan = -1
+        if seq_lens is not None:
+            _check(seq_lens.is_cuda and seq_lens.dtype == torch.int32
+                   and seq_lens.is_contiguous(), "seq_lens must be contiguous cuda int32")
+            _check(seq_lens.numel() == B, "seq_lens must have one entry per batch row")
+        if plan_lens is not None:
+            _check(seq_lens is not None, "plan_lens plans a ragged batch: seq_lens is required")
+            _check(len(plan_lens) == B, "plan_lens must have one entry per batch row")
+            plan = self.prefill_plan(plan_lens, T, H, pool.device, pool.dtype)
+        conv_out = torch.empty(B, T, C, device=x.device, dtype=torch.float32)
+        self._call("braid_gdn_conv_prefill_raw", pool.device, _ptr(pool), pdt, n_slots, H, G, SS,
+                   HD, _ptr(conv_pool), K, _ptr(slot_idx), B, T, _ptr(x), _ACT_DTYPES[x.dtype],
+                   _ptr(weight), bias_p, _ptr(conv_out), _ptr(a_raw), _ptr(b_raw), adt, _ptr(A),
+                   _ptr(dt_bias), _ptr(y), _ACT_DTYPES[y.dtype], _ptr(seq_lens), plan)
 
     def prefill_plan(self, lens: Sequence[int], T: int, H: int, device=None,
                      pool_dtype: torch.dtype = torch.float32) -> int:

@@ -11,9 +11,10 @@ here starts from their outputs: ``qkv_proj`` [B, T, C], ``z`` [B, T, H*HD]
 Differences from the reference's glue, each a consequence of kernels this
 build has and the reference had not:
 
-* prefill's causal conv runs ``conv1d_prefill`` (one launch, window saved in
-  place) instead of ``F.conv1d`` over ``[window | x]`` plus a gather
-  (gdn.py:193-222); outputs and windows equal ``conv1d_decode`` token by token;
+* prefill's causal conv runs as one launch (window saved in place) instead of
+  ``F.conv1d`` over ``[window | x]`` plus a gather (gdn.py:193-222); outputs and
+  windows equal ``conv1d_decode`` token by token. The scan reads q, k and v in
+  the conv's output as they lie (``gdn_conv_prefill_raw``);
 * decode runs the conv, the recurrence and the gated norm as one launch
   (``gdn_conv_decode_readout``) where the shape allows, instead of
   ``conv1d_decode`` then ``gdn_decode_raw`` (gdn.py:131-160) and the torch
@@ -120,18 +121,18 @@ class GDNMixerLayer:
         g = self.g
         if cache is None or slots_i32 is None:
             raise ValueError("a pooled cache needs a slot assignment")
-        B, T, C = qkv_proj.shape
+        B, T, _ = qkv_proj.shape
         lens = None if seq_lens is None else seq_lens.to(torch.int32).contiguous()
-        conv_out = torch.empty(B, T, C, device=qkv_proj.device, dtype=torch.float32)
-        self._mod.conv1d_prefill(cache.conv, slots_i32, qkv_proj.contiguous(), self.conv1d_f32,
-                                 self.conv_bias_f32, conv_out, lens)
-        q, k, v = self._split(conv_out)
+        a, b = a_raw.contiguous(), b_raw.contiguous()
+        # The readout rounds y to z's type first: where the scan can leave it
+        # rounded, half of y's bytes never move.
+        narrow = (z.dtype == a.dtype == torch.bfloat16 and cache.state.dtype != torch.float32)
         y = torch.empty(B, T, g.n_heads, g.head_dim, device=qkv_proj.device,
-                        dtype=torch.float32)
-        self._mod.gdn_prefill_raw(cache.state, slots_i32, q.contiguous(), k.contiguous(),
-                                  v.contiguous(), a_raw.contiguous(), b_raw.contiguous(),
-                                  self.A, self.dt_bias, y, lens,
-                                  plan_lens=plan_lens if lens is not None else None)
+                        dtype=torch.bfloat16 if narrow else torch.float32)
+        self._mod.gdn_conv_prefill_raw(cache.state, cache.conv, slots_i32, qkv_proj.contiguous(),
+                                       self.conv1d_f32, self.conv_bias_f32, a, b, self.A,
+                                       self.dt_bias, y, g.n_groups, lens,
+                                       plan_lens=plan_lens if lens is not None else None)
         return self._readout(z, y)
 
 

@@ -233,6 +233,26 @@ int braid_gdn_prefill_raw_plan(void* pool, int pool_dtype, int64_t n_slots, int 
                                float* y, const int32_t* seq_lens, int plan, void* stream);
 
 /*
+ * braid_conv1d_prefill followed by braid_gdn_prefill_raw_plan on the conv
+ * output's q/k/v columns, read in place, with one slot check: bit for bit the
+ * same y at live positions, pad zeros, state and windows.
+ *
+ *   conv_out  [B, T, C] fp32 scratch, C = 2*G*SS + H*HD; its live positions
+ *             hold the conv outputs afterwards, its pad positions anything
+ *   y         fp32, or (y_dtype BRAID_BF16: bf16 gates and a 16-bit pool) y
+ *             rounded to bf16, as braid_gated_rmsnorm_quant would round it
+ *   plan      as braid_gdn_prefill_raw_plan, < 0 for none
+ * Other arguments as the two calls'.
+ */
+int braid_gdn_conv_prefill_raw(void* pool, int pool_dtype, int64_t n_slots, int H, int G, int SS,
+                               int HD, float* conv_pool, int K, const int32_t* slot_idx, int B,
+                               int T, const void* x, int x_dtype, const float* conv_weight,
+                               const float* conv_bias, float* conv_out, const void* a_raw,
+                               const void* b_raw, int act_dtype, const float* A,
+                               const float* dt_bias, void* y, int y_dtype,
+                               const int32_t* seq_lens, int plan, void* stream);
+
+/*
  * Batched slotted causal depthwise conv1d, one decode step, SiLU fused.
  * Replaces conv1d_decode (braid/kernels/csrc/conv1d_decode.cu:91-149).
  *
