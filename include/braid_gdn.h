@@ -296,7 +296,8 @@ int braid_conv1d_prefill(float* conv_pool, int64_t n_slots, int C, int K,
 int braid_quantize_act_workspace(int64_t n);
 
 /*
- * Dynamic per-tensor FP8 e4m3fn activation quantization, two launches.
+ * Dynamic per-tensor FP8 e4m3fn activation quantization, two launches (one, with
+ * partial unused, for small inputs).
  * Replaces quantize_act (braid/kernels/csrc/quant_act.cu:140-176), which
  * allocated its outputs; here the caller passes them.
  *
