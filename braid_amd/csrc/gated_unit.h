@@ -114,6 +114,48 @@ __device__ __forceinline__ void gated_unit(float (&c)[4], const float (&zf)[4], 
   }
 }
 
+// The same unit on 16 lanes, eight consecutive elements each: a lane adds its two
+// quads, which the 32-lane butterfly's first stage adds across lanes, and the
+// other stages follow at half the distance, so the bits are gated_unit's.
+template <class ATag>
+__device__ __forceinline__ void gated_unit_wide(float (&c)[kVec], const float (&zf)[kVec],
+                                                const float (&gm)[kVec], float eps, bool live,
+                                                typename ATag::T* core, long i, float& m) {
+  uint32_t bits[kVec / 2];
+#pragma unroll
+  for (int e = 0; e < kVec; e += 2) Narrow<ATag>::pair(c[e], c[e + 1], bits[e / 2]);
+  float ss = ((c[0] * c[0] + c[1] * c[1]) + (c[2] * c[2] + c[3] * c[3])) +
+             ((c[4] * c[4] + c[5] * c[5]) + (c[6] * c[6] + c[7] * c[7]));
+  ss += lane_xor<1>(ss);
+  ss += lane_xor<2>(ss);
+  ss += lane_xor<4>(ss);
+  ss += lane_xor<8>(ss);
+  const float r = rsqrtf(ss * (1.0f / kUnit) + eps);
+  float o[kVec];
+#pragma unroll
+  for (int e = 0; e < kVec; ++e) o[e] = c[e] * r;
+#pragma unroll
+  for (int e = 0; e < kVec; e += 2) Narrow<ATag>::pair(o[e], o[e + 1], bits[e / 2]);
+#pragma unroll
+  for (int e = 0; e < kVec; ++e) {
+    const float h = gm[e] * o[e];
+    const float s = zf[e] / (1.0f + expf(-zf[e]));
+    o[e] = h * s;
+  }
+  if (live) {
+#pragma unroll
+    for (int e = 0; e < kVec; e += 2) Narrow<ATag>::pair(o[e], o[e + 1], bits[e / 2]);
+    if constexpr (sizeof(typename ATag::T) == 2) {
+      *reinterpret_cast<u32x4*>(core + i) = (u32x4){bits[0], bits[1], bits[2], bits[3]};
+    } else {
+      *reinterpret_cast<f32x4*>(core + i) = (f32x4){o[0], o[1], o[2], o[3]};
+      *reinterpret_cast<f32x4*>(core + i + 4) = (f32x4){o[4], o[5], o[6], o[7]};
+    }
+#pragma unroll
+    for (int e = 0; e < kVec; ++e) m = nan_max(m, fabsf(o[e]));
+  }
+}
+
 }  // namespace
 }  // namespace quant
 }  // namespace braid
