@@ -20,8 +20,9 @@ prebuilt gfx950 library ``braid_amd/libbraid_gdn.so`` (C ABI declared in
 Beyond the reference's six, the object fronts the rows this build adds on
 either side of the scan: ``conv1d_prefill`` (the prefill conv the reference
 ran in torch), ``gdn_conv_decode_raw`` (conv1d_decode + gdn_decode_raw in one
-launch), ``gated_rmsnorm`` (the readout and the out_proj input quantization)
-and ``fp8_matmul`` (the FP8 GEMM, hipBLASLt).
+launch), ``gated_rmsnorm`` (the readout and the out_proj input quantization),
+``gdn_conv_decode_readout`` and ``gdn_conv_prefill_raw`` (a layer's decode and
+prefill pieces joined) and ``fp8_matmul`` (the FP8 GEMM).
 
 There is no CPU or torch fallback: if the library is missing or a tensor is
 not on the GPU, the call raises.

@@ -8,14 +8,15 @@ decode launch goes on a second stream forked from the caller's, so the two
 kernels overlap: the prefill scan is a latency-bound serial chain (one
 workgroup per CU at a tick's sizes), and the decode, a memory stream, fills the
 CUs' remaining issue slots and the HBM beside it. On MI355X (config 4: 96
-decode rows + 4 x 256 prefill tokens, fp16 pool, graph-replayed) the tick takes
-129 us against 156 us in sequence; the prefill alone takes 119 us.
+decode rows + 4 x 256 prefill tokens, fp16 pool, graph-replayed) the tick takes 87 us
+(129 before the scan ran on the matrix cores, when the two in sequence took
+156 us and the prefill alone 119).
 
 The prefill is captured first, and that order matters: the graph's branches
 start in capture order, and a large decode asks for enough LDS to hold two of
 its workgroups per CU, so a decode that started first would keep the prefill's
-workgroups off the CUs until it drained (measured: 205 us for the tick with the
-decode captured first).
+workgroups off the CUs until it drained (205 us against 129 for the tick with the
+decode captured first, measured with the earlier scan).
 
 The two launches touch disjoint slots (the decode takes only rows that are no
 longer prefilling, scheduler.py:267), so their order does not change a bit:
