@@ -459,8 +459,9 @@ def measure_paths(torch, kern):
         plan_times = []
         for _ in range(5):
             t_plan = time.perf_counter()
-            plan = kern._lib.braid_prefill_plan(host.ctypes.data, Bp, T, H, cus)
+            plan = kern._lib.braid_prefill_plan_pool(host.ctypes.data, Bp, T, H, cus, 1)
             plan_times.append(time.perf_counter() - t_plan)
+        plan &= (1 << 28) - 1  # an fp16 pool's plan, without its mark
         n8, n4, n2 = plan >> 20, (plan >> 10) & 1023, plan & 1023
         # the launch an eager call makes: a launch small enough for the eighth
         # layout runs it without planning; one tier for every row runs that

@@ -1732,6 +1732,12 @@ int simulate_prefill16_plans(const std::vector<int>& lens, int H, int cus, const
   return plan;
 }
 
+// Marks a plan made for 16-bit pools (braid_prefill_plan_pool), so that a hint made
+// for the other kind's tier times shapes no launch: an fp32 pool's plan would
+// put one eighth-layout row on every CU ahead of fifteen short ones (0.337 ms
+// where the kernel's own estimate takes 0.264 and the right plan 0.236).
+constexpr int kPlan16 = 1 << 28;
+
 // Prefill layout of a launch on a 16-bit pool: the most workgroups per tile
 // that leave no CU with a second one (a token's time, one workgroup per CU:
 // eighth 0.160 us, quarter 0.172, split 0.250, whole 0.392, fp16), planned per
@@ -1772,7 +1778,8 @@ void launch_prefill16(void* pool, int pool_dtype, const int32_t* slot_idx, int B
   const bool chosen = plan < 0 && launch_knob(BRAID_KNOB_PREFILL_LAYOUT) < 0;
   if (chosen) plan = host_lens != nullptr
                          ? host_prefill_plan(*host_lens, T, H, some_cus, pool_dtype)
-                         : plan_hint;
+                         : (plan_hint >= 0 && (plan_hint & kPlan16) != 0 ? plan_hint & ~kPlan16
+                                                                         : -1);
   int max_extra = std::min(some_cus, 7 * B * H), n_wg = B * H + max_extra;
   if (plan >= 0) {
     const int n8 = std::min(plan >> 20, B), n4 = std::min((plan >> 10) & 1023, B - n8);
@@ -1822,7 +1829,7 @@ int launch_prefill(void* pool, int pool_dtype, const int32_t* slot_idx, int B, i
     host_plan = host_prefill_plan(*host_lens, T, H, cus);
     const int n8 = host_plan >> 20, n4 = (host_plan >> 10) & 1023, n2 = host_plan & 1023;
     layout = n8 == B ? 8 : (n4 == B ? 4 : (n2 == B ? 1 : 0));
-  } else if (plan_hint >= 0 && gates.ragged() && layout != 8 &&
+  } else if (plan_hint >= 0 && (plan_hint & kPlan16) == 0 && gates.ragged() && layout != 8 &&
              launch_knob(BRAID_KNOB_PREFILL_LAYOUT) < 0 &&
              launch_knob(BRAID_KNOB_PREFILL_PLAN) < 0 && B <= kMaxPlanRows && cus > 0 &&
              B * H <= 4 * cus) {
@@ -2250,7 +2257,8 @@ extern "C" int braid_prefill_plan_pool(const int32_t* seq_lens_host, int B, int 
     return -fail(BRAID_EINVAL,
                  "braid_prefill_plan_pool needs host lengths, B > 0, T >= 0, H > 0, cus > 0");
   return host_prefill_plan(std::vector<int32_t>(seq_lens_host, seq_lens_host + B), T, H, cus,
-                           pool_dtype);
+                           pool_dtype) |
+         (pool_dtype == BRAID_F32 ? 0 : kPlan16);
 }
 
 extern "C" int braid_prefill_plan(const int32_t* seq_lens_host, int B, int T, int H, int cus) {

@@ -452,8 +452,8 @@ class GDNKernels:
     def prefill_plan(self, lens: Sequence[int], T: int, H: int, device=None,
                      pool_dtype: torch.dtype = torch.float32) -> int:
         """The plan (n8 * 2^20 + n4 * 2^10 + n2) an eager ragged prefill of
-        these host lengths runs on ``device`` with a pool of ``pool_dtype``
-        (braid_prefill_plan_pool)."""
+        these host lengths runs on ``device`` with a pool of ``pool_dtype``,
+        plus 2^28 for a 16-bit pool (braid_prefill_plan_pool)."""
         cus = torch.cuda.get_device_properties(device).multi_processor_count
         arr = (ctypes.c_int32 * len(lens))(*[int(x) for x in lens])
         plan = self._lib.braid_prefill_plan_pool(ctypes.cast(arr, ctypes.c_void_p), len(lens), T,

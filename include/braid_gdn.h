@@ -92,8 +92,9 @@ enum braid_launch_knob {
 int braid_prefill_plan(const int32_t* seq_lens_host, int B, int T, int H, int cus);
 /*
  * The same for a pool of pool_dtype: a 16-bit pool's tiers have other times
- * (braid_prefill_plan is the fp32 pool's plan). Any plan suits any pool; this
- * one is what an eager call on such a pool chooses.
+ * (braid_prefill_plan is the fp32 pool's plan). This one is what an eager call
+ * on such a pool chooses, plus 2^28 for a 16-bit pool: a plan made for the other
+ * kind of pool is taken as none (the bits never depend on it).
  */
 int braid_prefill_plan_pool(const int32_t* seq_lens_host, int B, int T, int H, int cus,
                             int pool_dtype);
